@@ -252,6 +252,7 @@ int erod_batch_destroy(erod_batch* b) {
   }
   hipFree(b->d_time_next);
   for (double* p : b->d_shadow) hipFree(p);
+  hipFree(b->d_slot_rods);
   if (b->ev0) hipEventDestroy(b->ev0);
   if (b->ev1) hipEventDestroy(b->ev1);
   if (b->ev_fork) hipEventDestroy(b->ev_fork);
@@ -501,21 +502,7 @@ int erod_step(erod_batch* b, double* time, double dt, uint64_t n) {
   if (int rc = check_plain(b)) return rc;
   int rc = sync_rods(b);
   if (rc) return rc;
-  double t = *time;
-  for (uint64_t i = 0; i < n; ++i) {
-    if ((rc = ops_kinematic_update(b, dt))) return rc;
-    t += 0.5 * dt;
-    if ((rc = ops_apply_post_kinematic(b))) return rc;
-    if ((rc = ops_compute_internal_dynamics(b))) return rc;
-    if ((rc = ops_apply_pre_dynamic(b, t))) return rc;
-    if ((rc = ops_dynamic_update(b, dt))) return rc;
-    if ((rc = ops_apply_post_dynamic(b))) return rc;
-    t += 0.5 * dt;
-    if ((rc = ops_kinematic_update(b, dt))) return rc;
-  }
-  *time = t;
-  // every rod clock follows the caller's clock, so checkpoints carry it
-  return ops_set_rod_clocks(b, t);
+  return ops_step(b, time, dt, n);
 }
 
 int erod_set_rod_dt(erod_batch* b, const double* dt_per_rod) {

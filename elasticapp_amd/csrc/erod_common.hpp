@@ -189,8 +189,10 @@ struct erod_batch {
   // of reortho_every (0: never); reortho_phase = steps since the last one
   uint64_t reortho_every = 0, reortho_phase = 0;
   double* d_time_next = nullptr;  // rod clocks written by launches over pieces, copied back after each
-  // second copy of x, v, Q, w that launches over pieces alternate with (same layout as the fields)
+  // second copy of x, v, Q, w that launches over pieces, and launches of
+  // several op-by-op steps, alternate with (same layout as the fields)
   double* d_shadow[4] = {};
+  uint32_t* d_slot_rods = nullptr;  // rod of every slot, for the hooks of launches of several op-by-op steps
   // timing of the dominant kernel
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   // a second stream, and the events that fork a plan's tile groups onto it and
@@ -243,10 +245,11 @@ namespace erod {
   int ops_fill_ghosts(erod_batch* b, int field);
   int ops_mark_ghost_nodes(erod_batch* b);
   int ops_set_rod_clocks(erod_batch* b, double t);
+  // n whole steps; *time advances by n dt and every rod clock is set to it
+  int ops_step(erod_batch* b, double* time, double dt, uint64_t n);
   int ops_apply_post_kinematic(erod_batch* b);
   int ops_apply_pre_dynamic(erod_batch* b, double time);
   int ops_apply_post_dynamic(erod_batch* b);
-  int ops_zero_external(erod_batch* b);
   // fused path (erod_fused.hip)
   int fused_prepare(erod_batch* b, int precision);
   int fused_launch(erod_batch* b, int precision, int steps, bool timed);
