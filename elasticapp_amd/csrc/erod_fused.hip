@@ -582,7 +582,9 @@ namespace erod {
           rc = prc;
           break;
         }
-        if (prc != EROD_OK || b->plan.g[1].shape < 0) continue;  // infeasible here, or no second group
+        // infeasible here, or no second group, or every rod in it (a plan of
+        // that shape alone, which the first trials timed)
+        if (prc != EROD_OK || b->plan.g[1].shape < 0 || b->plan.g[0].shape < 0) continue;
         if ((rc = fused_launch(b, precision, trial_steps, false))) break;  // warm
         if ((rc = fused_launch(b, precision, trial_steps, true))) break;
         float ms = 0.0f;
