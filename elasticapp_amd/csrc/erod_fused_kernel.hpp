@@ -167,7 +167,7 @@ namespace erod {
       } else {
         const double th = sqrt(t2), r = 1.0 / t2;
         double s, c;
-        math::sincos(th, &s, &c);
+        math::sincos_any(th, &s, &c);
         A = s * th * r;
         B = (1.0 - c) * r;
       }
