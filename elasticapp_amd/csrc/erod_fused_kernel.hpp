@@ -540,7 +540,14 @@ namespace erod {
                                                   const uint32_t* __restrict__ tile_lane0, const Seg* __restrict__ segs,
                                                   const double* time_in, double* time_out, const uint32_t* steps_in,
                                                   uint32_t* steps_out, Env env, int nsteps, uint64_t E) {
-      constexpr bool kCache = sizeof(R) == 4;  // FP32 constants stay in registers for the launch
+      constexpr bool kCache = sizeof(R) == 4;  // FP32 constants stay in an LDS table for the launch
+      // FP64 at one element per thread: its constants stay in registers for the
+      // launch, so that no step waits for the 35 loads or forms their addresses.
+      // It takes fewer registers than reading them did (220 VGPRs, 245 before:
+      // the addresses go), and 1,024 rods of 64 elements 1.76 -> 1.65 ms per 500
+      // steps, 2,048 ragged rods 9.2 -> 8.9 ms per 300.  With more elements per
+      // thread there is no room, and they are read every step.
+      constexpr bool kHold = sizeof(R) == 8 && P == 1;
       // FP32-bulk: the closing half step of one step and the opening half step
       // of the next (same v and w) are taken as one update of dt within a launch
       constexpr bool kMerge = sizeof(R) == 4;
@@ -805,6 +812,17 @@ namespace erod {
         tail_gf = tail_m * tail_gf;
       }
       if constexpr (!kCache) __syncthreads();  // every lookup in the rod table done before s1 is written
+      ElemConst<R> H;  // kHold: the thread's element's constants
+      if constexpr (kHold) {
+        const uint64_t s = slot[0];
+        load_const<R>(C, s, E, !(kk[0] == nn[0] - 1) && !pad[0], H);
+#pragma unroll
+        for (int c = 0; c < 3; ++c) H.iJ[c] = C.iJ[c * E + s];
+        // the damping products, formed as every step would form them
+        gfj[0] = H.m * gfj[0];
+        gtj[0] = (R(0.5) * (H.m + H.mn)) * gtj[0];
+        tail_gf = tail_m * tail_gf;
+      }
       if (tid < 9) s3[tid][0] = R(0);  // read only after the barriers of the first step
       // whether a lane of this wave holds a clamped node or element: a
       // wave-uniform value, so that the waves without clamps (most of a
@@ -1016,6 +1034,8 @@ namespace erod {
             K.D0 = sc[kCache ? 11 : 0][kCache ? el : 0];
             K.il0 = inv_l0[kCache ? j : 0];
             K.iD0 = inv_D0[kCache ? j : 0];
+          } else if constexpr (kHold) {
+            K = H;
           } else {
             load_const<R>(C, slot[j], E, has_vor, K);
           }
@@ -1059,6 +1079,13 @@ namespace erod {
             im = inv_m[kCache ? j : 0];
 #pragma unroll
             for (int c = 0; c < 3; ++c) iJ[c] = inv_J[kCache ? j : 0][c];
+            mg = gfj[j];
+            eg = gtj[j];
+          } else if constexpr (kHold) {
+            mk = H.m;
+            im = H.invm;
+#pragma unroll
+            for (int c = 0; c < 3; ++c) iJ[c] = H.iJ[c];
             mg = gfj[j];
             eg = gtj[j];
           } else {
@@ -1115,7 +1142,7 @@ namespace erod {
           }
           // last node of the rod
           if (last) {
-            const R mgn = kCache ? tail_gf : tail_m * tail_gf;
+            const R mgn = kCache || kHold ? tail_gf : tail_m * tail_gf;
             double fen[3] = {0.0, 0.0, 0.0};
             if (rflags[j] & 2u) {
               if constexpr (kTailForce) {
