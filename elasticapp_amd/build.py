@@ -32,6 +32,7 @@ SOURCES = {
     "erod_capi.hip": [],
     "erod_serve.hip": [],
     "erod_io.hip": [],
+    "erod_xfer.hip": [],
 }
 
 

@@ -253,6 +253,7 @@ int erod_batch_destroy(erod_batch* b) {
   hipFree(b->d_time_next);
   for (double* p : b->d_shadow) hipFree(p);
   hipFree(b->d_slot_rods);
+  free_transfer_buffers(b);
   if (b->ev0) hipEventDestroy(b->ev0);
   if (b->ev1) hipEventDestroy(b->ev1);
   if (b->ev_fork) hipEventDestroy(b->ev_fork);
@@ -304,10 +305,7 @@ int erod_upload_field(erod_batch* b, int field, const double* host) {
 
 int erod_download_field(erod_batch* b, int field, double* host) {
   if (check_batch(b) || check_field(field) || !host) return EROD_ERR_INVALID;
-  const size_t bytes = sizeof(double) * field_info(field).ncomp * b->field_slots(field);
-  EROD_HIP(hipMemcpyAsync(host, b->d_field[field], bytes, hipMemcpyDeviceToHost, b->stream));
-  EROD_HIP(hipStreamSynchronize(b->stream));
-  return EROD_OK;
+  return download_lines(b, field, 0, b->field_slots(field), host);
 }
 
 static uint64_t rod_count(const erod_batch* b, int field, uint64_t rod) {
@@ -336,12 +334,7 @@ int erod_download_rod(erod_batch* b, int field, uint64_t rod, double* host) {
     set_error("erod_download_rod: bad argument (or an empty rod slot)");
     return EROD_ERR_INVALID;
   }
-  const uint64_t cnt = rod_count(b, field, rod), slots = b->field_slots(field), s = b->starts[rod];
-  const int nc = field_info(field).ncomp;
-  EROD_HIP(hipMemcpy2DAsync(host, cnt * sizeof(double), b->d_field[field] + s, slots * sizeof(double), cnt * sizeof(double),
-                            nc, hipMemcpyDeviceToHost, b->stream));
-  EROD_HIP(hipStreamSynchronize(b->stream));
-  return EROD_OK;
+  return download_lines(b, field, b->starts[rod], rod_count(b, field, rod), host);
 }
 
 int erod_fill_ghosts(erod_batch* b) {

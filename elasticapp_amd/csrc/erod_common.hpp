@@ -205,6 +205,10 @@ struct erod_batch {
   int* d_flags = nullptr;
   erod::CopyPair* d_copy_pairs = nullptr;  // grow-only staging of erod_copy_rods
   uint64_t copy_capacity = 0;
+  // pinned host memory of downloads (erod_xfer.hip), allocated on first use
+  void* stage = nullptr;  // small ones
+  void* ring = nullptr;   // large ones, a ring of chunks
+  hipEvent_t ring_ev[8] = {};
 
   uint64_t slots(int stagger) const { return stagger == EROD_NODE ? E + 1 : (stagger == EROD_ELEMENT ? E : E - 1); }
   uint64_t field_slots(int f) const { return slots(erod::field_info(f).stagger); }
@@ -263,6 +267,10 @@ namespace erod {
   // offset (in floats) of a field in the FP32 constant copy, or ~0 if the field
   // has none; valid while the copy is allocated and not dirty
   uint64_t fused_const32_offset(const erod_batch* b, int field);
+  // cnt values from `slot` on of every line of a field to host memory, line
+  // after line; returns when they are there
+  int download_lines(erod_batch* b, int field, uint64_t slot, uint64_t cnt, double* host);
+  void free_transfer_buffers(erod_batch* b);
   // device copy of whole rods between batches (admission of a request)
   int serve_copy_rods(erod_batch* dst, const erod_batch* src, const std::vector<CopyPair>& pairs);
   int fused_shape_lanes(int shape);
