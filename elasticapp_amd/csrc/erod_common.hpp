@@ -93,10 +93,15 @@ namespace erod {
   // A piece of a rod that one tile holds: elements [off, off + n) of rod
   // `rod`.  The tile writes back only the elements [off + w0, off + w1) it
   // owns (and their nodes); the others are a halo, the neighbouring pieces'
-  // elements, recomputed from the state they had when the launch began.  In
-  // one step a node or element depends on one neighbour before it and two
-  // after it, so a halo of h elements on each side keeps the owned elements
-  // exact for h / 2 steps: a launch over pieces takes at most that many.
+  // elements, recomputed from the state they had when the launch began.  What
+  // is wrong past a cut moves inward by one element a step.  On the left: the
+  // first element's -1 terms are wrong, hence after s steps nodes and elements
+  // below s.  On the right, where Q^T n / e of element k needs nodes k, k + 1
+  // and director k, and the couple of region k nodes up to k + 2 and director
+  // k + 1: the piece's last node and its last element's torque are wrong after
+  // one step, and after s steps nodes from n - s + 1 and elements from n - s on.
+  // So a halo of h elements on each side keeps the owned elements exact for h
+  // steps: a launch over pieces takes at most that many.
   // `ends`: kSegFirst if the piece starts at the rod's first element,
   // kSegLast if it ends at the rod's last (the rod end rules, clamp and end
   // force apply only at such ends).
@@ -119,6 +124,7 @@ namespace erod {
     uint32_t* d_seg_rods = nullptr;    // the rods cut into the pieces
     uint64_t n_seg_rods = 0, seg_rod_capacity = 0;
     int max_steps = 0;                 // steps per launch at most (0: no limit)
+    int run_steps = 0;                 // pieces: steps of a run within a launch (k_fused's split)
   };
 
   struct FusedPlan {

@@ -525,7 +525,7 @@ namespace erod {
     // kEnv: 0 no environment, 1 gravity and / or contact with a level plane,
     // 2 contact with a plane of any normal
     //
-    // The entries of a tile are whole rods, or, with `segs`, pieces of rods
+    // The entries of a tile are whole rods, or, with kSegs, pieces of rods
     // (Seg): a piece runs as a rod of its own length whose elements outside
     // [w0, w1) are not written back, and whose cut ends take the rod-end
     // rules with neither clamp nor end force (its halo absorbs the error).
@@ -534,12 +534,16 @@ namespace erod {
     // rods the same arrays; over pieces, which share their rod's clock and
     // budget across tiles, the clock goes to a second array (from the piece
     // holding the rod's last element) and the budget is spent after the launch.
-    template <typename R, int P, int NT, int kEnv>
+    // A launch takes `total` steps; over pieces, FP32-bulk ends a run of
+    // `split` of them with the closing half step and opens the next with one of
+    // its own, as if it were a launch of its own (so that its results do not
+    // depend on how many runs a launch holds).
+    template <typename R, int P, int NT, int kEnv, bool kSegs>
     __global__ void __launch_bounds__(NT) k_fused(StatePtrs in, StatePtrs out, Consts<R> C, const RodInfo* __restrict__ rods,
                                                   const Tile* __restrict__ tiles, const uint32_t* __restrict__ tile_rods,
                                                   const uint32_t* __restrict__ tile_lane0, const Seg* __restrict__ segs,
                                                   const double* time_in, double* time_out, const uint32_t* steps_in,
-                                                  uint32_t* steps_out, Env env, int nsteps, uint64_t E) {
+                                                  uint32_t* steps_out, Env env, int total, int split, uint64_t E) {
       constexpr bool kCache = sizeof(R) == 4;  // FP32 constants stay in an LDS table for the launch
       // FP64 at one element per thread: its constants stay in registers for the
       // launch, so that no step waits for the 35 loads or forms their addresses.
@@ -647,7 +651,7 @@ namespace erod {
         e_[j] = find(uint32_t(tid) * P + j);
         const uint32_t ent = t_rod[e_[j]];
         uint32_t r;
-        if (segs) {
+        if constexpr (kSegs) {
           const Seg sg = segs[ent];
           r = sg.rod;
           s_off[j] = sg.off;
@@ -677,8 +681,8 @@ namespace erod {
 #pragma unroll
       for (int j = 0; j < P; ++j) {
         const uint32_t el = uint32_t(tid) * P + j, e = e_[j];
-        const uint32_t segn = segs ? s_n[j] : r_n[j], off = s_off[j], ends = s_ends[j];
-        const uint32_t w0 = s_w0[j], w1 = segs ? s_w1[j] : segn;
+        const uint32_t segn = kSegs ? s_n[j] : r_n[j], off = s_off[j], ends = s_ends[j];
+        const uint32_t w0 = s_w0[j], w1 = kSegs ? s_w1[j] : segn;
         const uint32_t padn = (uint32_t(P) - segn % uint32_t(P)) % uint32_t(P), raw = el - t_lane0[e];
         pad[j] = el < tile.lanes && raw < padn;
         valid[j] = el < tile.lanes && raw >= padn;
@@ -697,7 +701,7 @@ namespace erod {
           if ((i < r_n[j] ? i : r_n[j] - 1) == g) rflags[j] |= uint32_t(k + 1) << 12;
         }
         own[j] = valid[j] && uint32_t(kk[j]) >= w0 && uint32_t(kk[j]) < w1;
-        clockw[j] = valid[j] && kk[j] == 0 && (segs == nullptr || (ends & kSegLast) != 0);
+        clockw[j] = valid[j] && kk[j] == 0 && (!kSegs || (ends & kSegLast) != 0);
         if (j == P - 1 && valid[j] && kk[j] == int(segn) - 1) tailw = (ends & kSegLast) != 0;
         // damping rates: one per rod, or (flag bit 2) per node and element
         const bool per_node = (r_fl[j] & 4u) != 0 && valid[j];
@@ -844,6 +848,8 @@ namespace erod {
         lim[j] = valid[j] ? lim[j] : 0u;
       }
       asm volatile("" : "+v"(wb));
+      constexpr bool kRuns = kSegs && kMerge;
+      int nsteps = kRuns && split < total ? split : total, rest = total - nsteps;
       for (int step = 0; step < nsteps; ++step) {
         // a rod whose budget is spent keeps its state (its element forces are
         // still evaluated, since the tile moves in lockstep, but never applied)
@@ -1208,6 +1214,15 @@ namespace erod {
 #pragma unroll
             for (int c = 0; c < 3; ++c) xt[c] = maddd<R>(ch, vt[c], xt[c]);
         }
+        if (kRuns && step + 1 == nsteps && rest > 0) {
+          // the next run of steps
+#pragma unroll
+          for (int j = 0; j < P; ++j)
+            if (lim[j] != kNoBudget) lim[j] = lim[j] > uint32_t(nsteps) ? lim[j] - uint32_t(nsteps) : 0u;
+          nsteps = split < rest ? split : rest;
+          rest -= nsteps;
+          step = -1;
+        }
       }
 
       // ---- write back (one field line at a time over the P elements) --------------
@@ -1247,18 +1262,21 @@ namespace erod {
         }
         if ((wb >> (8 + j)) & 1u) {
           time_out[rodi[j]] = tm[j];
-          if (steps_out && lim[j] != kNoBudget) steps_out[rodi[j]] = lim[j] > uint32_t(nsteps) ? lim[j] - uint32_t(nsteps) : 0u;
+          if (!kSegs && steps_out && lim[j] != kNoBudget)
+            steps_out[rodi[j]] = lim[j] > uint32_t(total) ? lim[j] - uint32_t(total) : 0u;
         }
       }
     }
 
     // the state of the rods cut into pieces, from the second copy back into
-    // the fields (after an odd number of launches over pieces); one
-    // workgroup per rod
+    // the fields (after an odd number of launches over pieces), and, when
+    // time_from is set, their clocks; one workgroup per rod
     static __global__ void k_copy_cut_state(const uint32_t* __restrict__ seg_rods, const RodInfo* __restrict__ rods,
-                                            StatePtrs from, StatePtrs to, uint64_t E) {
+                                            StatePtrs from, StatePtrs to, const double* __restrict__ time_from,
+                                            double* __restrict__ time_to, uint64_t E) {
       const uint64_t N = E + 1;
       const RodInfo ri = rods[seg_rods[blockIdx.x]];
+      if (time_from && threadIdx.x == 0) time_to[seg_rods[blockIdx.x]] = time_from[seg_rods[blockIdx.x]];
       for (uint32_t k = threadIdx.x; k <= ri.n; k += blockDim.x) {
         const uint64_t s = ri.start + k;
         for (int c = 0; c < 3; ++c) {
@@ -1294,21 +1312,27 @@ namespace erod {
       return StatePtrs{b->d_shadow[0], b->d_shadow[1], b->d_shadow[2], b->d_shadow[3]};
     }
 
+    // the two clocks arrays a launch reads and writes (for whole rods the same)
+    struct Clocks {
+      double *in, *out;
+    };
+
     template <typename R, int P, int NT, int kEnv>
     inline void launch_env(erod_batch* b, const Consts<R>& C, int steps, const TileGroup& g, const StatePtrs& in,
-                           const StatePtrs& out, hipStream_t st) {
+                           const StatePtrs& out, const Clocks& t, hipStream_t st) {
       uint32_t* budgets = b->budgets ? b->d_steps_left : nullptr;
       if (g.d_segs) {
-        // pieces: clocks to the second array, budgets spent afterwards
-        hipLaunchKernelGGL((k_fused<R, P, NT, kEnv>), dim3(static_cast<unsigned>(g.n_tiles)), dim3(NT), 0, st, in,
-                           out, C, b->d_rods, g.d_tiles, g.d_tile_rods, g.d_tile_lane0, g.d_segs, b->d_time, b->d_time_next,
-                           budgets, nullptr, b->env, steps, b->E);
-        hipLaunchKernelGGL(k_seg_clocks, dim3(static_cast<unsigned>((g.n_seg_rods + 255) / 256)), dim3(256), 0, st,
-                           g.d_seg_rods, g.n_seg_rods, b->d_time_next, b->d_time, budgets, uint32_t(steps));
+        hipLaunchKernelGGL((k_fused<R, P, NT, kEnv, true>), dim3(static_cast<unsigned>(g.n_tiles)), dim3(NT), 0, st, in,
+                           out, C, b->d_rods, g.d_tiles, g.d_tile_rods, g.d_tile_lane0, g.d_segs, t.in, t.out,
+                           budgets, nullptr, b->env, steps, g.run_steps, b->E);
+        // budgets are spent after the launch, the clocks then copied back
+        if (budgets)
+          hipLaunchKernelGGL(k_seg_clocks, dim3(static_cast<unsigned>((g.n_seg_rods + 255) / 256)), dim3(256), 0, st,
+                             g.d_seg_rods, g.n_seg_rods, t.out, t.in, budgets, uint32_t(steps));
       } else {
-        hipLaunchKernelGGL((k_fused<R, P, NT, kEnv>), dim3(static_cast<unsigned>(g.n_tiles)), dim3(NT), 0, st, in,
-                           out, C, b->d_rods, g.d_tiles, g.d_tile_rods, g.d_tile_lane0, nullptr, b->d_time, b->d_time,
-                           budgets, budgets, b->env, steps, b->E);
+        hipLaunchKernelGGL((k_fused<R, P, NT, kEnv, false>), dim3(static_cast<unsigned>(g.n_tiles)), dim3(NT), 0, st, in,
+                           out, C, b->d_rods, g.d_tiles, g.d_tile_rods, g.d_tile_lane0, nullptr, t.in, t.out,
+                           budgets, budgets, b->env, steps, steps, b->E);
       }
     }
 
@@ -1317,13 +1341,13 @@ namespace erod {
     // plane runs one without the arithmetic of a general normal
     template <typename R, int P, int NT>
     inline int launch_tiles(erod_batch* b, const Consts<R>& C, int steps, const TileGroup& g, const StatePtrs& in,
-                            const StatePtrs& out, hipStream_t st) {
+                            const StatePtrs& out, const Clocks& t, hipStream_t st) {
       if (g.n_tiles == 0) return EROD_OK;
       const Env& e = b->env;
       const bool level = e.n[0] == 0.0 && e.n[1] == 0.0 && e.n[2] == 1.0;
-      if (e.contact && !level) launch_env<R, P, NT, 2>(b, C, steps, g, in, out, st);
-      else if (e.gravity || e.contact) launch_env<R, P, NT, 1>(b, C, steps, g, in, out, st);
-      else launch_env<R, P, NT, 0>(b, C, steps, g, in, out, st);
+      if (e.contact && !level) launch_env<R, P, NT, 2>(b, C, steps, g, in, out, t, st);
+      else if (e.gravity || e.contact) launch_env<R, P, NT, 1>(b, C, steps, g, in, out, t, st);
+      else launch_env<R, P, NT, 0>(b, C, steps, g, in, out, t, st);
       return hip_check(hipGetLastError(), "k_fused");
     }
 
@@ -1336,16 +1360,16 @@ namespace erod {
 
     template <typename R>
     inline int launch_shape(erod_batch* b, const Consts<R>& C, int steps, int shape, const TileGroup& g,
-                            const StatePtrs& in, const StatePtrs& out, hipStream_t st) {
+                            const StatePtrs& in, const StatePtrs& out, const Clocks& t, hipStream_t st) {
       switch (shape) {
-        case 0: return launch_tiles<R, 1, 64>(b, C, steps, g, in, out, st);
-        case 1: return launch_tiles<R, 1, 128>(b, C, steps, g, in, out, st);
-        case 2: return launch_tiles<R, 1, 256>(b, C, steps, g, in, out, st);
-        case 3: return launch_tiles<R, 1, 512>(b, C, steps, g, in, out, st);
-        case 4: return launch_tiles<R, 2, 256>(b, C, steps, g, in, out, st);
-        case 5: return launch_tiles<R, 2, 512>(b, C, steps, g, in, out, st);
-        case 6: return launch_tiles<R, 4, 128>(b, C, steps, g, in, out, st);
-        case 7: return launch_tiles<R, 4, 256>(b, C, steps, g, in, out, st);
+        case 0: return launch_tiles<R, 1, 64>(b, C, steps, g, in, out, t, st);
+        case 1: return launch_tiles<R, 1, 128>(b, C, steps, g, in, out, t, st);
+        case 2: return launch_tiles<R, 1, 256>(b, C, steps, g, in, out, t, st);
+        case 3: return launch_tiles<R, 1, 512>(b, C, steps, g, in, out, t, st);
+        case 4: return launch_tiles<R, 2, 256>(b, C, steps, g, in, out, t, st);
+        case 5: return launch_tiles<R, 2, 512>(b, C, steps, g, in, out, t, st);
+        case 6: return launch_tiles<R, 4, 128>(b, C, steps, g, in, out, t, st);
+        case 7: return launch_tiles<R, 4, 256>(b, C, steps, g, in, out, t, st);
         default: set_error("bad tile shape"); return EROD_ERR_INVALID;
       }
     }
@@ -1357,23 +1381,25 @@ namespace erod {
     inline int launch_group(erod_batch* b, const Consts<R>& C, int steps, const TileGroup& g, hipStream_t st) {
       if (g.shape < 0 || g.n_tiles == 0) return EROD_OK;
       const StatePtrs fields = field_state(b);
-      if (!g.d_segs) return launch_shape(b, C, steps, g.shape, g, fields, fields, st);
+      if (!g.d_segs) return launch_shape(b, C, steps, g.shape, g, fields, fields, Clocks{b->d_time, b->d_time}, st);
       // pieces: launches of at most max_steps steps, each reading the state
-      // the previous one wrote and writing the other copy; the state ends in
-      // the fields
+      // (and, unless budgets are spent between them, the clocks) the previous
+      // one wrote and writing the other copy; the state ends in the fields
       const StatePtrs shadow = shadow_state(b);
       const int cap = g.max_steps > 0 ? g.max_steps : steps;
       bool in_fields = true;
       for (int done = 0; done < steps;) {
         const int s = steps - done < cap ? steps - done : cap;
-        if (int rc = launch_shape(b, C, s, g.shape, g, in_fields ? fields : shadow, in_fields ? shadow : fields, st))
+        const bool back = !in_fields && !b->budgets;
+        const Clocks t{back ? b->d_time_next : b->d_time, back ? b->d_time : b->d_time_next};
+        if (int rc = launch_shape(b, C, s, g.shape, g, in_fields ? fields : shadow, in_fields ? shadow : fields, t, st))
           return rc;
         in_fields = !in_fields;
         done += s;
       }
       if (!in_fields) {
         hipLaunchKernelGGL(k_copy_cut_state, dim3(static_cast<unsigned>(g.n_seg_rods)), dim3(256), 0, st, g.d_seg_rods,
-                           b->d_rods, shadow, fields, b->E);
+                           b->d_rods, shadow, fields, b->budgets ? nullptr : b->d_time_next, b->d_time, b->E);
         return hip_check(hipGetLastError(), "k_copy_cut_state");
       }
       return EROD_OK;

@@ -194,8 +194,9 @@ int erod_get_fused_split(const erod_batch* b, int* lanes_per_tile, int* elements
  * elements_per_thread 0 = either): each piece owns a part of its rod and
  * recomputes `halo` elements (0 = 16, at least 2) of each neighbouring piece
  * from the state they had when the launch began, so that pieces need no
- * exchange within a launch; a launch over pieces then takes at most halo / 2
- * steps, and the pieces' group is launched as often as needed.  Results do
+ * exchange within a launch; a launch over pieces then takes at most halo (or
+ * halo - 1, if odd) steps, and the pieces' group is launched as often as
+ * needed.  Results do
  * not depend on the cut (bitwise).  For rods longer than any tile (the
  * reference's blocks emplace rods of any length, Block.hpp:568-611) and for
  * fused FP64, whose long-rod tiles spill registers.  The getter reports the
