@@ -175,6 +175,7 @@ int erod_batch_create(const uint64_t* n_elems, uint64_t n_rods, int damped, erod
   EROD_HIP(hipGetDevice(&device));
   auto* b = new erod_batch();
   b->device = device;
+  if (hipDeviceGetAttribute(&b->cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || b->cus <= 0) b->cus = 256;
   b->n_rods = n_rods;
   b->damped = damped != 0;
   b->n_elems.assign(n_elems, n_elems + n_rods);
@@ -243,13 +244,14 @@ int erod_batch_destroy(erod_batch* b) {
   hipFree(b->d_time);
   hipFree(b->d_flags);
   hipFree(b->d_const32);
-  for (TileGroup& g : b->plan.g) {
-    hipFree(g.d_tiles);
-    hipFree(g.d_tile_rods);
-    hipFree(g.d_tile_lane0);
-    hipFree(g.d_segs);
-    hipFree(g.d_seg_rods);
-  }
+  for (TileGroup* set : {b->plan.g, b->plan.kept.g})
+    for (TileGroup* g = set; g != set + 3; ++g) {
+      hipFree(g->d_tiles);
+      hipFree(g->d_tile_rods);
+      hipFree(g->d_tile_lane0);
+      hipFree(g->d_segs);
+      hipFree(g->d_seg_rods);
+    }
   hipFree(b->d_time_next);
   for (double* p : b->d_shadow) hipFree(p);
   hipFree(b->d_slot_rods);

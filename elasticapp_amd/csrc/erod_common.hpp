@@ -142,12 +142,22 @@ namespace erod {
     // groups: 0 main, 1 second (short rods), 2 pieces of long rods
     TileGroup g[3];
     bool valid = false;
+    // where the caller leaves the shapes free they depend on the precision:
+    // the precision, main shape and pieces' shape of g, and the plan of the
+    // other precision, kept while both are in use
+    int precision = -1, main_shape = -1, piece_shape = -1;
+    struct Kept {
+      TileGroup g[3];
+      bool valid = false;
+      int main_shape = -1, piece_shape = -1;
+    } kept;
   };
 
 }  // namespace erod
 
 struct erod_batch {
   int device = 0;
+  int cus = 256;  // compute units of the device
   hipStream_t stream = nullptr;
   uint64_t n_rods = 0;
   uint64_t E = 0;  // element slots incl. ghosts

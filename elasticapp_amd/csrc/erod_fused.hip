@@ -109,16 +109,6 @@ namespace erod {
     return b->n_active[r] != 0 && (!b->budgets || b->steps_left[r] != 0);
   }
 
-  // the shape of the pieces of long rods: the one of seg_lanes lanes (and
-  // seg_epl elements per thread when set), or the main shape; -2 if none
-  static int piece_shape(const erod_batch* b, int main_shape) {
-    if (b->plan.seg_lanes <= 0) return main_shape;
-    for (int si : {0, 1, 2, 4, 5, 3, 7, 6})  // the default order of preference
-      if (fused_shape_lanes(si) == b->plan.seg_lanes && (b->plan.seg_epl <= 0 || fused_shape_epl(si) == b->plan.seg_epl))
-        return si;
-    return -2;
-  }
-
   // A rod runs as pieces when it is longer than the main tile, or longer
   // than the pieces' tile when seg_lanes is set.
   static bool cut_rod(const erod_batch* b, uint64_t n, int main_shape) {
@@ -139,27 +129,74 @@ namespace erod {
     return true;
   }
 
+  // whether neither the caller nor the autotuner chose the main shape
+  static bool shapes_free(const erod_batch* b) {
+    return b->plan.lanes_per_tile == 0 && b->plan.elements_per_thread == 0 && b->plan.tuned_shape < 0;
+  }
+
+  constexpr int kShape256 = 2, kShape512 = 3;  // one element per thread
+
   // Default shape without measurement: the smallest capacity that holds the
   // longest rod; one element per thread up to 256 lanes, two elements per
-  // thread for 512 and 1024 lanes; rods longer than 1024 elements run as
-  // pieces.  (FP32-bulk on ragged batches: 512 lanes at two elements per
-  // thread, two 4-wave workgroups per CU, run 27% faster than one element
-  // per thread in 8-wave workgroups; four elements per thread spill and run
-  // one wave per SIMD.)  A shape the autotuner chose is taken again while it
-  // stays feasible (a replan after rods changed length keeps it, with its
-  // second group).
-  static int default_shape(const erod_batch* b) {
+  // thread for 1024 lanes; rods longer than 1024 elements run as pieces.  (Four
+  // elements per thread spill and run one wave per SIMD.)  512 lanes take two
+  // elements per thread for FP32-bulk when the tiles fill more than a round of
+  // the CUs: two 4-wave workgroups share a CU (1,200 rods of 16 to 512
+  // elements: 3.6 us a step against 4.4 in 8-wave workgroups of one element per
+  // thread).  While every tile has a CU of its own a step costs its latency,
+  // which is shorter at one element per thread (600 such rods: 2.40 against
+  // 2.65; 61 rods of up to 301: 2.15 against 2.67); fused FP64 has no registers
+  // for two (17.5 against 21.0 for 2,400 rods, 5.7 against 7.1 for 61).
+  // A shape the autotuner chose is taken again while it stays feasible (a
+  // replan after rods changed length keeps it, with its second group).
+  static int default_shape(const erod_batch* b, int precision) {
     static const int pref[] = {0, 1, 2, 4, 5, 3, 7, 6};
     if (b->plan.tuned_shape >= 0 && shape_feasible(b, b->plan.tuned_shape)) return b->plan.tuned_shape;
-    uint64_t maxn = 0;
+    uint64_t maxn = 0, lanes = 0;
     for (uint64_t r = 0; r < b->n_rods; ++r)
-      if (planned(b, r)) maxn = std::max<uint64_t>(maxn, b->n_active[r]);
+      if (planned(b, r)) {
+        maxn = std::max<uint64_t>(maxn, b->n_active[r]);
+        lanes += b->n_active[r];
+      }
     for (int si : pref)
-      if (uint64_t(fused_shape_lanes(si)) >= maxn && shape_feasible(b, si)) return si;
+      if (uint64_t(fused_shape_lanes(si)) >= maxn && shape_feasible(b, si)) {
+        const bool two = fused_shape_lanes(si) == 512 && fused_shape_epl(si) == 2;
+        if (two && shape_feasible(b, kShape512) && (precision == EROD_FP64 || lanes <= 512 * uint64_t(b->cus))) return kShape512;
+        return si;
+      }
     // longer rods than any tile: the largest tiles, the longer rods in pieces
     for (int si : {5, 4, 3, 2, 1, 0, 7, 6})
       if (shape_feasible(b, si)) return si;
     return -1;
+  }
+
+  // The shape of the pieces of long rods: the one of seg_lanes lanes (and
+  // seg_epl elements per thread when set), or the main shape; -2 if none.
+  // With every shape free, smaller pieces than the main tiles where those
+  // would leave CUs idle, and always for fused FP64, whose 1024-lane tiles
+  // spill registers.  24 rods of 2,500 to 6,000 elements (107 / 212 / 440
+  // pieces of 1024 / 512 / 256 lanes on 256 CUs), us a step: FP32-bulk 6.0 /
+  // 4.4 / 4.5, FP64 21.1 / 7.7 / 8.2; 2 rods of 1,200 to 1,500: 4.6 / 3.2 / 2.7
+  // and 14.8 / 6.5 / 4.5; 60 rods of 1,100 to 6,000 (206 / 391 / 803): 6.4 / 7.3
+  // / 7.0 and 22.8 / 13.7 / 13.1.
+  static int piece_shape(const erod_batch* b, int main_shape, int precision) {
+    if (b->plan.seg_lanes > 0) {
+      for (int si : {0, 1, 2, 4, 5, 3, 7, 6})  // the default order of preference
+        if (fused_shape_lanes(si) == b->plan.seg_lanes && (b->plan.seg_epl <= 0 || fused_shape_epl(si) == b->plan.seg_epl))
+          return si;
+      return -2;
+    }
+    const uint64_t halo = uint64_t(b->plan.halo);
+    if (!shapes_free(b) || fused_shape_lanes(main_shape) != 1024 || 2 * halo + 64 > 256) return main_shape;
+    uint64_t pieces256 = 0, pieces512 = 0;
+    for (uint64_t r = 0; r < b->n_rods; ++r)
+      if (planned(b, r) && cut_rod(b, b->n_active[r], main_shape)) {
+        pieces256 += (b->n_active[r] + 255 - 2 * halo) / (256 - 2 * halo);
+        pieces512 += (b->n_active[r] + 511 - 2 * halo) / (512 - 2 * halo);
+      }
+    if (pieces256 <= uint64_t(b->cus)) return kShape256;
+    if (pieces512 <= uint64_t(b->cus)) return kShape512;
+    return precision == EROD_FP64 ? kShape256 : main_shape;
   }
 
   // One group of tiles on the host: the tiles, their entries (rods or
@@ -331,9 +368,8 @@ namespace erod {
     return -2;
   }
 
-  static int plan_tiles(erod_batch* b, int si) {
+  static int plan_tiles(erod_batch* b, int si, int ps, int precision) {
     const uint64_t cap = uint64_t(fused_shape_lanes(si));
-    const int ps = piece_shape(b, si);
     if (ps == -2) {
       set_error("plan_tiles: no tile shape of the requested piece lanes and elements per thread");
       return EROD_ERR_INVALID;
@@ -436,6 +472,9 @@ namespace erod {
     gs.run_steps = int(halo / 2);
     gs.max_steps = 2 * gs.run_steps;
     if (segs.empty()) gs.shape = -1;
+    pl.precision = precision;
+    pl.main_shape = si;
+    pl.piece_shape = ps;
     pl.valid = true;
     b->graph_precision = -1;
     return EROD_OK;
@@ -444,14 +483,26 @@ namespace erod {
   int fused_prepare(erod_batch* b, int precision) {
     int rc = sync_rods(b);
     if (rc) return rc;
-    if (!b->plan.valid) {
-      const int si = default_shape(b);
+    FusedPlan& pl = b->plan;
+    if (!pl.valid) pl.kept.valid = false;  // the rods changed: so did its
+    if (!pl.valid || pl.precision != precision) {
+      const int si = default_shape(b, precision);
       if (si < 0) {
         set_error("no fused tile shape holds this batch (a requested shape with more elements per thread than "
                   "a rod has)");
         return EROD_ERR_UNSUPPORTED;
       }
-      if ((rc = plan_tiles(b, si))) return rc;
+      const int ps = piece_shape(b, si, precision);
+      if (pl.valid && (si != pl.main_shape || ps != pl.piece_shape)) {
+        // the other precision's shapes: its plan comes in, this one is kept
+        for (int k = 0; k < 3; ++k) std::swap(pl.g[k], pl.kept.g[k]);
+        std::swap(pl.main_shape, pl.kept.main_shape);
+        std::swap(pl.piece_shape, pl.kept.piece_shape);
+        std::swap(pl.valid, pl.kept.valid);
+        pl.valid = pl.valid && pl.main_shape == si && pl.piece_shape == ps;
+      }
+      if (!pl.valid && (rc = plan_tiles(b, si, ps, precision))) return rc;
+      pl.precision = precision;
     }
     if (precision == EROD_FP32_BULK && b->const32_dirty) {
       const uint64_t total = const32_offset(b, kNConst32);
@@ -558,11 +609,14 @@ namespace erod {
     b->plan.lanes_per_tile = 0;
     b->plan.elements_per_thread = 0;
     b->budgets = false;  // trial launches leave the step budgets alone
+    // pieces of the requested shape, or of the main one
+    auto tuned_pieces = [&](int si) { return b->plan.seg_lanes > 0 ? piece_shape(b, si, precision) : si; };
+    b->plan.kept.valid = false;
     int best = -1;
     double best_t = 0.0;
     for (int si = 0; si < fused::kNShapes && rc == EROD_OK; ++si) {
       if (!shape_feasible(b, si)) continue;
-      if ((rc = plan_tiles(b, si))) break;
+      if ((rc = plan_tiles(b, si, tuned_pieces(si), precision))) break;
       if ((rc = fused_launch(b, precision, trial_steps, false))) break;  // warm
       if ((rc = fused_launch(b, precision, trial_steps, true))) break;
       float ms = 0.0f;
@@ -582,7 +636,7 @@ namespace erod {
         if (fused_shape_lanes(s2) >= cap) continue;
         b->plan.split_lanes = fused_shape_lanes(s2);
         b->plan.split_epl = fused_shape_epl(s2);
-        const int prc = plan_tiles(b, best);
+        const int prc = plan_tiles(b, best, tuned_pieces(best), precision);
         if (prc == EROD_ERR_HIP) {  // a device failure ends the search; an infeasible shape does not
           rc = prc;
           break;
@@ -611,7 +665,7 @@ namespace erod {
     b->plan.split_epl = best_split >= 0 ? fused_shape_epl(best_split) : g.split_epl;
     g.keep_split = true;
     b->budgets = g.budgets;
-    if (rc == EROD_OK && best >= 0) rc = plan_tiles(b, best);
+    if (rc == EROD_OK && best >= 0) rc = plan_tiles(b, best, tuned_pieces(best), precision);
     if (rc == EROD_OK) rc = restore();
     if (rc == EROD_OK) rc = hip_check(hipStreamSynchronize(b->stream), "autotune");
     if (rc == EROD_OK && best < 0) {

@@ -176,8 +176,10 @@ int erod_set_rod_time(erod_batch* b, const double* time_per_rod);
  * steps_per_launch: steps a workgroup advances with its rods' state held on
  * chip (0 = 100).  The rods of a batch share one shape.  Without a request or
  * an autotune, a batch takes the smallest capacity that holds its longest rod
- * (one element per thread up to 256 lanes, two from 512); rods longer than
- * the tile run as pieces (erod_set_fused_pieces). */
+ * (one element per thread up to 256 lanes, two from 1024; at 512 two for
+ * FP32-bulk batches of more tiles than the device has compute units, one
+ * otherwise); rods longer than the tile run as pieces
+ * (erod_set_fused_pieces).  Results do not depend on the shape. */
 int erod_set_fused_config(erod_batch* b, int lanes_per_tile, int elements_per_thread, int steps_per_launch);
 int erod_get_fused_config(const erod_batch* b, int* lanes_per_tile, int* elements_per_thread, int* steps_per_launch);
 /* A second group of tiles: a rod of at most lanes_per_tile elements that finds
@@ -190,14 +192,15 @@ int erod_get_fused_config(const erod_batch* b, int* lanes_per_tile, int* element
 int erod_set_fused_split(erod_batch* b, int lanes_per_tile, int elements_per_thread);
 int erod_get_fused_split(const erod_batch* b, int* lanes_per_tile, int* elements_per_thread, uint64_t* tiles);
 /* Rods longer than the main tile, or longer than lanes_per_tile when it is
- * not 0, run as pieces in tiles of that shape (0: the main shape;
- * elements_per_thread 0 = either): each piece owns a part of its rod and
+ * not 0, run as pieces in tiles of that shape (0: the main shape, or, when no
+ * shape was requested or tuned, smaller tiles where those leave fewer compute
+ * units idle, and 256 lanes for FP64; elements_per_thread 0 = either): each
+ * piece owns a part of its rod and
  * recomputes `halo` elements (0 = 16, at least 2) of each neighbouring piece
  * from the state they had when the launch began, so that pieces need no
  * exchange within a launch; a launch over pieces then takes at most halo (or
  * halo - 1, if odd) steps, and the pieces' group is launched as often as
- * needed.  Results do
- * not depend on the cut (bitwise).  For rods longer than any tile (the
+ * needed.  Results do not depend on the cut (bitwise).  For rods longer than any tile (the
  * reference's blocks emplace rods of any length, Block.hpp:568-611) and for
  * fused FP64, whose long-rod tiles spill registers.  The getter reports the
  * pieces' shape, halo, tiles and pieces in the current plan (0 if none). */
