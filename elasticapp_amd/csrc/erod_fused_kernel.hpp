@@ -545,13 +545,16 @@ namespace erod {
                                                   const double* time_in, double* time_out, const uint32_t* steps_in,
                                                   uint32_t* steps_out, Env env, int total, int split, uint64_t E) {
       constexpr bool kCache = sizeof(R) == 4;  // FP32 constants stay in an LDS table for the launch
-      // FP64 at one element per thread: its constants stay in registers for the
-      // launch, so that no step waits for the 35 loads or forms their addresses.
-      // It takes fewer registers than reading them did (220 VGPRs, 245 before:
-      // the addresses go), and 1,024 rods of 64 elements 1.76 -> 1.65 ms per 500
-      // steps, 2,048 ragged rods 9.2 -> 8.9 ms per 300.  With more elements per
-      // thread there is no room, and they are read every step.
-      constexpr bool kHold = sizeof(R) == 8 && P == 1;
+      // One element per thread: its constants stay in registers for the launch.
+      // FP64 would wait for 35 loads and form their addresses every step, and
+      // takes fewer registers without them (220 VGPRs, 245 before): 1,024 rods
+      // of 64 elements 1.76 -> 1.65 ms per 500 steps, 2,048 ragged rods 9.2 ->
+      // 8.9 ms per 300.  FP32-bulk would read the LDS table (18 words a step;
+      // 173 VGPRs, 167 before): us a step 1.26 -> 1.22 for 64 rods of 64, 1.51
+      // -> 1.47 for 1,024, 3.57 -> 3.06 for 3,072, 7.5 -> 6.9 for 8,192, 15.1 ->
+      // 14.7 for 8,192 of 128 with contact.  With more elements per thread there
+      // is no room: FP64 reads them every step, FP32-bulk from the table.
+      constexpr bool kHold = P == 1;
       // FP32-bulk: the closing half step of one step and the opening half step
       // of the next (same v and w) are taken as one update of dt within a launch
       constexpr bool kMerge = sizeof(R) == 4;
@@ -817,7 +820,21 @@ namespace erod {
       }
       if constexpr (!kCache) __syncthreads();  // every lookup in the rod table done before s1 is written
       ElemConst<R> H;  // kHold: the thread's element's constants
-      if constexpr (kHold) {
+      if constexpr (kHold && kCache) {
+        H.l0 = sc[1][tid];
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+          H.sig0[c] = sc[kCache ? 2 + c : 0][tid];
+          H.S[c] = sc[kCache ? 5 + c : 0][tid];
+          H.J[c] = sc[kCache ? 8 + c : 0][tid];
+          H.kap0[c] = sc[kCache ? 12 + c : 0][tid];
+          H.B[c] = sc[kCache ? 15 + c : 0][tid];
+        }
+        H.D0 = sc[kCache ? 11 : 0][tid];
+        H.il0 = inv_l0[0];
+        H.iD0 = inv_D0[0];
+        H.m = sc[0][tid];
+      } else if constexpr (kHold) {
         const uint64_t s = slot[0];
         load_const<R>(C, s, E, !(kk[0] == nn[0] - 1) && !pad[0], H);
 #pragma unroll
@@ -1026,7 +1043,9 @@ namespace erod {
             }
           }
           ElemConst<R> K;
-          if constexpr (kCache) {
+          if constexpr (kHold) {
+            K = H;
+          } else if constexpr (kCache) {
             const uint32_t el = uint32_t(j) * NT + tid;  // lane tid P + j
             K.l0 = sc[1][el];
 #pragma unroll
@@ -1040,8 +1059,6 @@ namespace erod {
             K.D0 = sc[kCache ? 11 : 0][kCache ? el : 0];
             K.il0 = inv_l0[kCache ? j : 0];
             K.iD0 = inv_D0[kCache ? j : 0];
-          } else if constexpr (kHold) {
-            K = H;
           } else {
             load_const<R>(C, slot[j], E, has_vor, K);
           }
@@ -1081,7 +1098,7 @@ namespace erod {
           R mk, im, iJ[3], mg, eg;
           if constexpr (kCache) {
             // (the mass itself only for the environment's loads)
-            mk = kEnv != 0 ? sc[0][uint32_t(j) * NT + tid] : R(0);
+            mk = kEnv != 0 ? (kHold ? H.m : sc[0][uint32_t(j) * NT + tid]) : R(0);
             im = inv_m[kCache ? j : 0];
 #pragma unroll
             for (int c = 0; c < 3; ++c) iJ[c] = inv_J[kCache ? j : 0][c];
