@@ -224,7 +224,7 @@ struct erod_batch {
   // pinned host memory of downloads (erod_xfer.hip), allocated on first use
   void* stage = nullptr;  // small ones
   void* ring = nullptr;   // large ones, a ring of chunks
-  hipEvent_t ring_ev[8] = {};
+  hipEvent_t ring_ev[4] = {};
 
   uint64_t slots(int stagger) const { return stagger == EROD_NODE ? E + 1 : (stagger == EROD_ELEMENT ? E : E - 1); }
   uint64_t field_slots(int f) const { return slots(erod::field_info(f).stagger); }

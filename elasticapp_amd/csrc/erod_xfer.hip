@@ -7,17 +7,19 @@
 //   - what is below kRingFrom goes to pinned memory of the batch in one copy, a
 //     rod's lines packed by a kernel that writes it directly, and from there
 //     to the caller: 12 us for a few KB, strided or not, 25 us for 350 KB (26
-//     or 156 before, by where the caller's memory lies), 58 us for 1 MB;
-//   - beyond, a ring of pinned chunks fills on the batch's stream while the
-//     full ones are copied out by two threads, from 4 MB on by four, so that
-//     page faults and host copies run side by side: 28 MB 1.63 -> 0.93 ms, 72 MB
-//     of fresh memory 7.0 -> 2.5 ms.  Eight threads were slower than four, and
-//     chunks below 1 MB slower too (each copy costs 14 us whatever its size);
+//     or 156 before, by where the caller's memory lies);
+//   - beyond, a ring of pinned chunks fills from the batch's two streams while
+//     two threads, from 2 MB on four, copy the full ones out, so that page
+//     faults and host copies run side by side: 24 MB 1.41 -> 0.59 ms, 72 MB of
+//     fresh memory 7.0 -> 2.5 ms.  Six and eight threads were not faster.  A
+//     copy costs 14 us beside its bytes, whatever its size, which the other
+//     stream's copy hides (0.66 ms on one stream); chunks of 2 MB against 1 MB:
+//     0.65 and 0.80 ms on one stream;
 //   - longer strided lines, and whatever finds no pinned memory, are copied as
 //     before.
+#include <algorithm>
 #include <atomic>
 #include <cstring>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -27,8 +29,8 @@ namespace erod {
 
   namespace {
     constexpr size_t kStageBytes = size_t(256) << 10;
-    constexpr size_t kRingFrom = size_t(2) << 20, kChunk = size_t(1) << 20;
-    constexpr int kRing = 8;  // chunks in the ring
+    constexpr size_t kRingFrom = size_t(1) << 20, kChunk = size_t(2) << 20;
+    constexpr int kRing = 4;  // chunks in the ring
     constexpr int kThreadsMost = 4;
 
     // lines of cnt values, `pitch` apart, one after another into pinned memory
@@ -59,36 +61,44 @@ namespace erod {
     // `bytes` from device memory into the caller's through the ring.  The
     // calling thread makes every HIP call: it queues a chunk's copy once the
     // slot's last content has been copied out, waits for copies in order and
-    // publishes how many have landed; the threads (it among them) take the
-    // landed chunks in turn.
+    // publishes how many have landed; every thread (it among them) copies its
+    // share of each landed chunk.  Chunks go alternately to the batch's two
+    // streams, so that one is in flight while the other's copy starts or ends.
     int download_ring(erod_batch* b, const char* src, char* host, size_t bytes) {
-      const size_t want = bytes < (size_t(4) << 20) ? 2 : kThreadsMost;
-      const size_t chunks = (bytes + kChunk - 1) / kChunk;
+      const size_t mb = size_t(1) << 20, want = bytes < 2 * mb ? 2 : kThreadsMost;
+      const size_t chunk = bytes < 6 * mb ? kChunk / 2 : kChunk;
+      const size_t chunks = (bytes + chunk - 1) / chunk;
       char* ring = static_cast<char*>(b->ring);
-      auto size_of = [&](size_t i) { return i + 1 < chunks ? kChunk : bytes - i * kChunk; };
+      auto size_of = [&](size_t i) { return i + 1 < chunks ? chunk : bytes - i * chunk; };
       auto queue = [&](size_t i) -> int {
-        EROD_HIP(hipMemcpyAsync(ring + (i % kRing) * kChunk, src + i * kChunk, size_of(i), hipMemcpyDeviceToHost, b->stream));
-        EROD_HIP(hipEventRecord(b->ring_ev[i % kRing], b->stream));
+        hipStream_t st = (i & 1) ? b->stream2 : b->stream;
+        EROD_HIP(hipMemcpyAsync(ring + (i % kRing) * chunk, src + i * chunk, size_of(i), hipMemcpyDeviceToHost, st));
+        EROD_HIP(hipEventRecord(b->ring_ev[i % kRing], st));
         return EROD_OK;
       };
+      // the second stream starts after the work already queued on the first
+      EROD_HIP(hipEventRecord(b->ev_fork, b->stream));
+      EROD_HIP(hipStreamWaitEvent(b->stream2, b->ev_fork, 0));
       std::atomic<size_t> landed{0};
       std::atomic<bool> stop{false};
-      // chunk i is copied out by thread i mod n; each thread counts its own
-      std::atomic<size_t> out[kThreadsMost];
+      std::atomic<size_t> out[kThreadsMost];  // chunks each thread has copied its share of
       for (auto& o : out) o.store(0);
       std::vector<std::thread> helpers;
       std::atomic<size_t> n_threads{0};  // known once the helpers are up
-      auto copy_out = [&](size_t i) { std::memcpy(host + i * kChunk, ring + (i % kRing) * kChunk, size_of(i)); };
+      auto copy_out = [&](size_t i, size_t k, size_t n) {
+        const size_t size = size_of(i), part = ((size + n - 1) / n + 63) / 64 * 64, lo = std::min(size, k * part);
+        std::memcpy(host + i * chunk + lo, ring + (i % kRing) * chunk + lo, std::min(size, lo + part) - lo);
+        out[k].store(i + 1, std::memory_order_release);
+      };
       auto help = [&](size_t k) {
-        while (n_threads.load(std::memory_order_acquire) == 0) std::this_thread::yield();
-        const size_t n = n_threads.load(std::memory_order_acquire);
-        for (size_t i = k; i < chunks; i += n) {
+        size_t n;
+        while ((n = n_threads.load(std::memory_order_acquire)) == 0) std::this_thread::yield();
+        for (size_t i = 0; i < chunks; ++i) {
           while (landed.load(std::memory_order_acquire) <= i) {
             if (stop.load(std::memory_order_acquire)) return;
             std::this_thread::yield();
           }
-          copy_out(i);
-          out[k].fetch_add(1, std::memory_order_release);
+          copy_out(i, k, n);
         }
       };
       size_t queued = 0;
@@ -102,18 +112,21 @@ namespace erod {
       }
       const size_t n = helpers.size() + 1;
       n_threads.store(n, std::memory_order_release);
+      // whether every thread is done with chunk i
+      auto copied = [&](size_t i) {
+        for (size_t k = 0; k < n; ++k)
+          if (out[k].load(std::memory_order_acquire) <= i) return false;
+        return true;
+      };
       for (size_t i = 0; i < chunks && rc == EROD_OK; ++i) {
         rc = hip_check(hipEventSynchronize(b->ring_ev[i % kRing]), "download");
         if (rc) break;
         landed.store(i + 1, std::memory_order_release);
-        if (i % n == 0) {
-          copy_out(i);
-          out[0].fetch_add(1, std::memory_order_release);
-        }
-        // the oldest slot is free again when its chunk is out
+        copy_out(i, 0, n);
+        // a slot is free again when its chunk is out
         while (queued < chunks && rc == EROD_OK) {
           const size_t old = queued - kRing;
-          if (old > i || out[old % n].load(std::memory_order_acquire) <= old / n) {
+          if (old > i || !copied(old)) {
             if (queued > i + 1) break;  // others are still in flight: look again after the next one lands
             std::this_thread::yield();
             continue;
@@ -124,7 +137,10 @@ namespace erod {
       }
       if (rc) stop.store(true, std::memory_order_release);
       for (std::thread& t : helpers) t.join();
-      if (rc) (void)hipStreamSynchronize(b->stream);
+      if (rc) {
+        (void)hipStreamSynchronize(b->stream2);
+        (void)hipStreamSynchronize(b->stream);
+      }
       return rc;
     }
   }  // namespace

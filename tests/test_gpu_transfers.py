@@ -1,7 +1,7 @@
 """Downloads return what was uploaded, bit for bit, at the sizes where their
-path changes: the pinned stages (to 256 KB and 2 MB), the ring of 1 MB chunks
-(two threads, from 4 MB four; past its 8 chunks), whole fields and strided
-rods.
+path changes: the pinned stages (to 256 KB and 1 MB), the ring of chunks (two
+threads, from 2 MB four; 1 MB chunks, from 6 MB 2 MB; past its 4 chunks),
+whole fields and strided rods.
 """
 import threading
 
@@ -27,8 +27,8 @@ def _check(blk, rng, rounds=2):
 
 
 # Position at 24 B a slot: 256 KB at 10,922 slots, 1 MB at 43,690; Director at
-# 72 B: 2 MB at 29,127, whole chunks and one value more, and rings that wrap
-@pytest.mark.parametrize("n", [2, 10921, 10922, 29127, 29128, 43690, 58254, 58255, 116508, 116509, 131071, 131072, 300001])
+# 72 B: 1 MB at 14,563, 2 MB at 29,127, whole chunks and one value more, and rings that wrap
+@pytest.mark.parametrize("n", [2, 10921, 10922, 14563, 14564, 29127, 29128, 43690, 58254, 58255, 116508, 116509, 131071, 131072, 300001])
 def test_one_rod(n):
     with DeviceBlock([n]) as blk:
         _check(blk, np.random.default_rng(n))
