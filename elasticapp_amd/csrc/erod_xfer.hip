@@ -17,10 +17,14 @@
 //     0.65 and 0.80 ms on one stream;
 //   - longer strided lines, and whatever finds no pinned memory, are copied as
 //     before.
+#include <sys/mman.h>
+#include <unistd.h>
+
 #include <algorithm>
 #include <atomic>
 #include <cstring>
 #include <thread>
+#include <utility>
 #include <vector>
 
 #include "erod_common.hpp"
@@ -58,6 +62,30 @@ namespace erod {
       return EROD_OK;
     }
 
+    // The caller's pages in [p, p + n) that are about to be written, made
+    // present in one call if some are not: faulted in one by one by the copy
+    // they halve its rate (1.6 MB of fresh memory by one thread 0.32 ms, 0.16
+    // with this; a pass that keeps eight fields of 1.6 to 4.8 MB 2.5 -> 2.1 ms).
+    // Asking costs nothing that can be measured, and what the system refuses
+    // the copy does by itself.  Not for four threads: they fault beside each
+    // other, and eight fields of 6 to 18 MB took 5.4 ms with it, 5.0 without.
+    void make_present(char* p, size_t n) {
+#if defined(MADV_POPULATE_WRITE)
+      static const size_t page = size_t(sysconf(_SC_PAGESIZE));
+      const uintptr_t lo = (reinterpret_cast<uintptr_t>(p) + page - 1) / page * page;
+      const uintptr_t hi = (reinterpret_cast<uintptr_t>(p) + n) / page * page;
+      unsigned char in[512];
+      if (hi <= lo || (hi - lo) / page < 16 || (hi - lo) / page > sizeof(in)) return;
+      void* const at = reinterpret_cast<void*>(lo);
+      if (mincore(at, hi - lo, in) != 0) return;
+      for (size_t i = 0; i < (hi - lo) / page; ++i)
+        if (!(in[i] & 1)) {
+          (void)madvise(at, hi - lo, MADV_POPULATE_WRITE);
+          return;
+        }
+#endif
+    }
+
     // `bytes` from device memory into the caller's through the ring.  The
     // calling thread makes every HIP call: it queues a chunk's copy once the
     // slot's last content has been copied out, waits for copies in order and
@@ -85,15 +113,26 @@ namespace erod {
       for (auto& o : out) o.store(0);
       std::vector<std::thread> helpers;
       std::atomic<size_t> n_threads{0};  // known once the helpers are up
-      auto copy_out = [&](size_t i, size_t k, size_t n) {
+      // thread k's share of chunk i: [first, first + second)
+      auto share = [&](size_t i, size_t k, size_t n) {
         const size_t size = size_of(i), part = ((size + n - 1) / n + 63) / 64 * 64, lo = std::min(size, k * part);
-        std::memcpy(host + i * chunk + lo, ring + (i % kRing) * chunk + lo, std::min(size, lo + part) - lo);
+        return std::pair<size_t, size_t>(lo, std::min(size, lo + part) - lo);
+      };
+      auto ready = [&](size_t i, size_t k, size_t n) {
+        if (n > 2) return;
+        const auto [lo, len] = share(i, k, n);
+        make_present(host + i * chunk + lo, len);
+      };
+      auto copy_out = [&](size_t i, size_t k, size_t n) {
+        const auto [lo, len] = share(i, k, n);
+        std::memcpy(host + i * chunk + lo, ring + (i % kRing) * chunk + lo, len);
         out[k].store(i + 1, std::memory_order_release);
       };
       auto help = [&](size_t k) {
         size_t n;
         while ((n = n_threads.load(std::memory_order_acquire)) == 0) std::this_thread::yield();
         for (size_t i = 0; i < chunks; ++i) {
+          ready(i, k, n);
           while (landed.load(std::memory_order_acquire) <= i) {
             if (stop.load(std::memory_order_acquire)) return;
             std::this_thread::yield();
@@ -119,6 +158,7 @@ namespace erod {
         return true;
       };
       for (size_t i = 0; i < chunks && rc == EROD_OK; ++i) {
+        ready(i, 0, n);
         rc = hip_check(hipEventSynchronize(b->ring_ev[i % kRing]), "download");
         if (rc) break;
         landed.store(i + 1, std::memory_order_release);
@@ -160,6 +200,7 @@ namespace erod {
                            b->stream, src, slots, cnt, nc, static_cast<double*>(stage));
         EROD_HIP(hipGetLastError());
       }
+      make_present(reinterpret_cast<char*>(host), bytes);  // (while the copy is under way)
       EROD_HIP(hipStreamSynchronize(b->stream));
       std::memcpy(host, stage, bytes);
       return EROD_OK;
