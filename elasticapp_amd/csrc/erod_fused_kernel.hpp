@@ -50,6 +50,8 @@
 //   kinematic update of dt.
 #pragma once
 
+#include <type_traits>
+
 #include "erod_common.hpp"
 #include "erod_math.hpp"
 #include "erod_step64.hpp"
@@ -99,7 +101,6 @@ namespace erod {
                                        (__attribute__((address_space(3))) void*)wave_dst, 4, 0, 0);
     }
     __device__ __forceinline__ float sqrt_(float x) { return __builtin_amdgcn_sqrtf(x); }
-    __device__ __forceinline__ double sqrt_(double x) { return sqrt(x); }
 
     // a * b + c: one fused multiply-add in the FP32-bulk path, a separately
     // rounded product and sum in the FP64 path (which keeps the reference's
@@ -113,14 +114,6 @@ namespace erod {
     }
     __device__ __forceinline__ float madd(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
     __device__ __forceinline__ double madd(double a, double b, double c) { return a * b + c; }
-
-    // element length from an FP64 node difference; both neighbours of a
-    // Voronoi region evaluate it the same way
-    template <typename R>
-    __device__ __forceinline__ R len_(double d0, double d1, double d2) {
-      if constexpr (sizeof(R) == 8) return sqrt(d0 * d0 + d1 * d1 + d2 * d2);
-      else return sqrt_(static_cast<float>(__builtin_fma(d2, d2, __builtin_fma(d1, d1, d0 * d0))));
-    }
 
     // FP32 length of an FP32 difference
     __device__ __forceinline__ float len32(float a, float b, float c) { return sqrt_(madd(c, c, madd(b, b, a * a))); }
@@ -188,15 +181,6 @@ namespace erod {
 
     // ---- curvature of the Voronoi region between directors qc and qn / D0 --------
 
-    template <typename R>
-    __device__ __forceinline__ void curvature(const double qc[9], const double qn[9], R D0, R kap[3]);
-
-    // the reference's formula
-    template <>
-    __device__ __forceinline__ void curvature<double>(const double qc[9], const double qn[9], double D0, double kap[3]) {
-      step64::curvature(qc, qn, D0, kap);
-    }
-
     // FP32-bulk: skew part and trace in FP64, prefactor in FP32.  With
     // a = sin^2(theta/2) (3 - tr)/4 + 5e-11, the reference prefactor
     // theta / (2 sin theta) equals asin(sqrt a) / (2 sqrt(a) sqrt(1 - a)),
@@ -215,8 +199,7 @@ namespace erod {
       return __builtin_fma(-c[2], d[2], s);
     }
 
-    template <>
-    __device__ __forceinline__ void curvature<float>(const double qc[9], const double qn[9], float iD0, float kap[3]) {
+    __device__ __forceinline__ void curvature32(const double qc[9], const double qn[9], float iD0, float kap[3]) {
       const double tr = dot3_fma(qc, qn) + dot3_fma(qc + 3, qn + 3) + dot3_fma(qc + 6, qn + 6);
       // rows: d1 = q[0..2], d2 = q[3..5], d3 = q[6..8]
       const double s0 = skew3_fma(qc + 6, qn + 3, qc + 3, qn + 6);
@@ -255,7 +238,7 @@ namespace erod {
       R m, invm, mn;  // node k mass and inverse, node k+1 mass
       R l0, sig0[3], S[3], J[3], iJ[3];
       R D0, kap0[3], B[3];  // Voronoi k (unused at the rod end)
-      R il0, iD0;           // 1 / l0, 1 / D0 (FP32-bulk only)
+      R il0, iD0;           // 1 / l0, 1 / D0 (FP64: of step64::divisor, with kHold)
     };
 
     template <typename R>
@@ -303,13 +286,19 @@ namespace erod {
 
     // Element k (and Voronoi k when it exists) of a rod: everything that needs
     // only the +1 / +2 neighbours.  qr is the director used for Q t and Q^T n
-    // (the FP64 state for R = double, its FP32 copy for R = float).
-    template <typename R>
+    // (the FP64 state for R = double, its FP32 copy for R = float).  kPlain
+    // (FP64): divisions and roots without their special cases, `range` noting
+    // whether the operands allowed that.
+    template <typename R, bool kPlain = false>
     __device__ __forceinline__ void element_forces(const double xk[3], const double xk1[3], const double xk2[3],
                                                    const float dn[3], const double vk[3], const double vk1[3],
                                                    const double qk[9], const R qr[9], const double qk1[9],
                                                    const double wk[3], bool has_vor, const ElemConst<R>& K,
-                                                   Mid<R>& out, const float* geo = nullptr) {
+                                                   Mid<R>& out, const float* geo = nullptr,
+                                                   step64::Range* range = nullptr) {
+      using step64::Divisor;
+      using step64::divisor;
+      using step64::over;
       // spanwise geometry.  FP64: the reference's node difference, length and
       // tangent.  FP32-bulk: the node difference in FP64 rounded to FP32, then
       // everything in FP32; an element's length is a function of that rounded
@@ -320,10 +309,17 @@ namespace erod {
       R l, t[3];
       if constexpr (sizeof(R) == 8) {
         const double d0 = xk1[0] - xk[0], d1 = xk1[1] - xk[1], d2 = xk1[2] - xk[2];
-        l = len_<R>(d0, d1, d2);
-        t[0] = d0 / l;
-        t[1] = d1 / l;
-        t[2] = d2 / l;
+        l = step64::root<kPlain>(d0 * d0 + d1 * d1 + d2 * d2);
+        const Divisor by = divisor<kPlain>(l);
+        t[0] = over<kPlain>(d0, by);
+        t[1] = over<kPlain>(d1, by);
+        t[2] = over<kPlain>(d2, by);
+        if constexpr (kPlain) {
+          range->divisor(l);
+          range->numerator(d0);
+          range->numerator(d1);
+          range->numerator(d2);
+        }
       } else {
         const float d0 = geo ? geo[0] : static_cast<float>(xk1[0] - xk[0]),
                     d1 = geo ? geo[1] : static_cast<float>(xk1[1] - xk[1]),
@@ -335,8 +331,11 @@ namespace erod {
         t[2] = d2 * il;
       }
       R e, ie;
+      Divisor bye;
       if constexpr (sizeof(R) == 8) {
-        e = l / K.l0;
+        e = over<kPlain>(l, Divisor{K.l0, K.il0});
+        bye = divisor<kPlain>(e);
+        if constexpr (kPlain) range->divisor(e);
         ie = R(0);
       } else {
         e = l * K.il0;
@@ -358,7 +357,7 @@ namespace erod {
       for (int j = 0; j < 3; ++j) qn[j] = madd(qr[6 + j], n[2], madd(qr[3 + j], n[1], qr[j] * n[0]));
       if constexpr (sizeof(R) == 8) {
 #pragma unroll
-        for (int j = 0; j < 3; ++j) out.c[j] = qn[j] / e;
+        for (int j = 0; j < 3; ++j) out.c[j] = over<kPlain>(qn[j], bye);
       } else {
 #pragma unroll
         for (int j = 0; j < 3; ++j) out.c[j] = qn[j] * ie;
@@ -371,8 +370,21 @@ namespace erod {
       R jw[3];
 #pragma unroll
       for (int c = 0; c < 3; ++c) {
-        if constexpr (sizeof(R) == 8) jw[c] = (K.J[c] * w[c]) / e;
-        else jw[c] = (K.J[c] * w[c]) * ie;
+        if constexpr (sizeof(R) == 8) {
+          jw[c] = K.J[c] * w[c];
+          if constexpr (kPlain) {
+            range->numerator(qn[c]);
+            range->numerator(jw[c]);
+          }
+        } else {
+          jw[c] = (K.J[c] * w[c]) * ie;
+        }
+      }
+      if constexpr (sizeof(R) == 8) {
+        if constexpr (kPlain)
+          range->largest(((fabs(qn[0]) + fabs(qn[1])) + (fabs(qn[2]) + fabs(jw[0]))) + (fabs(jw[1]) + fabs(jw[2])));
+#pragma unroll
+        for (int c = 0; c < 3; ++c) jw[c] = over<kPlain>(jw[c], bye);
       }
       R lag[3];
       cross3(jw, w, lag);
@@ -400,7 +412,8 @@ namespace erod {
         R l1;
         if constexpr (sizeof(R) == 8) {
           const double f0 = xk2[0] - xk1[0], f1 = xk2[1] - xk1[1], f2 = xk2[2] - xk1[2];
-          l1 = len_<R>(f0, f1, f2);
+          l1 = step64::root<kPlain>(f0 * f0 + f1 * f1 + f2 * f2);
+          if constexpr (kPlain) range->divisor(l1);
         } else {
           l1 = geo ? geo[4] : len32(dn[0], dn[1], dn[2]);
         }
@@ -408,16 +421,24 @@ namespace erod {
         R eps;
         R kap[3];
         if constexpr (sizeof(R) == 8) {
-          eps = D / K.D0;
-          curvature<R>(qk, qk1, K.D0, kap);
+          const Divisor D0{K.D0, K.iD0};
+          eps = over<kPlain>(D, D0);
+          step64::curvature<kPlain>(qk, qk1, D0, kap);
         } else {
           eps = D * K.iD0;
-          curvature<R>(qk, qk1, K.iD0, kap);
+          curvature32(qk, qk1, K.iD0, kap);
         }
         R M[3];
 #pragma unroll
         for (int c = 0; c < 3; ++c) M[c] = K.B[c] * (kap[c] - K.kap0[c]);
-        const R ic = rcp_(eps * eps * eps);
+        R ic;
+        if constexpr (sizeof(R) == 8) {
+          const double cube = eps * eps * eps;
+          ic = over<kPlain>(1.0, divisor<kPlain>(cube));
+          if constexpr (kPlain) range->divisor(cube);
+        } else {
+          ic = rcp_(eps * eps * eps);
+        }
         R km[3];
         cross3(kap, M, km);
         const R icd = ic * K.D0;
@@ -555,6 +576,7 @@ namespace erod {
       // 14.7 for 8,192 of 128 with contact.  With more elements per thread there
       // is no room: FP64 reads them every step, FP32-bulk from the table.
       constexpr bool kHold = P == 1;
+      constexpr bool kPlainFirst = kHold && !kCache;
       // FP32-bulk: the closing half step of one step and the opening half step
       // of the next (same v and w) are taken as one update of dt within a launch
       constexpr bool kMerge = sizeof(R) == 4;
@@ -839,10 +861,17 @@ namespace erod {
         load_const<R>(C, s, E, !(kk[0] == nn[0] - 1) && !pad[0], H);
 #pragma unroll
         for (int c = 0; c < 3; ++c) H.iJ[c] = C.iJ[c * E + s];
+        H.il0 = step64::divisor<true>(H.l0).r;
+        H.iD0 = step64::divisor<true>(H.D0).r;
         // the damping products, formed as every step would form them
         gfj[0] = H.m * gfj[0];
         gtj[0] = (R(0.5) * (H.m + H.mn)) * gtj[0];
         tail_gf = tail_m * tail_gf;
+      }
+      step64::Range consts;  // whether the constants allow plain divisions
+      if constexpr (kPlainFirst) {
+        consts.divisor(H.l0);
+        consts.divisor(H.D0);
       }
       if (tid < 9) s3[tid][0] = R(0);  // read only after the barriers of the first step
       // whether a lane of this wave holds a clamped node or element: a
@@ -866,7 +895,12 @@ namespace erod {
       }
       asm volatile("" : "+v"(wb));
       constexpr bool kRuns = kSegs && kMerge;
-      int nsteps = kRuns && split < total ? split : total, rest = total - nsteps;
+      int nsteps = kRuns && split < total ? split : total;
+      // (what the end of a run needs, at one element per thread in vector
+      // registers: the loop has none of the scalar ones to spare, and 24 rods of
+      // 2,500 to 6,000 elements took 3.76 us a step instead of 3.63)
+      int run = split, rest = total - nsteps;
+      if constexpr (kRuns && P == 1) asm volatile("" : "+v"(run), "+v"(rest));
       for (int step = 0; step < nsteps; ++step) {
         // a rod whose budget is spent keeps its state (its element forces are
         // still evaluated, since the tile moves in lockstep, but never applied)
@@ -977,71 +1011,72 @@ namespace erod {
             continue;
           }
           const bool last = j == P - 1 && kk[j] == nn[j] - 1;
-          double xk1[3], xk2[3] = {0, 0, 0}, vk1[3], qk1[9];
-          float dn[3] = {0.0f, 0.0f, 0.0f};
-          if (last) {
-#pragma unroll
-            for (int c = 0; c < 3; ++c) {
-              xk1[c] = xt[c];
-              vk1[c] = vt[c];
-            }
-          } else if (j + 1 < P) {
-#pragma unroll
-            for (int c = 0; c < 3; ++c) {
-              xk1[c] = x[j + 1 < P ? j + 1 : j][c];
-              vk1[c] = v[j + 1 < P ? j + 1 : j][c];
-            }
-          } else {
-#pragma unroll
-            for (int c = 0; c < 3; ++c) {
-              xk1[c] = s1[c][tn];
-              vk1[c] = s1[3 + c][tn];
-            }
-          }
           const bool has_vor = !last && !pad[j];
-          // the next lane's director and node difference; for a rod's last
-          // element they belong to the next rod (or to an idle lane: identity
-          // director, zero state) and only meet its zero Voronoi constants
-          // (FP32-bulk) or are not used (FP64)
-          {
-            if (j + 1 < P) {
+          // the values of the next lanes
+          auto load_next = [&](double (&xk1)[3], double (&xk2)[3], double (&vk1)[3], double (&qk1)[9], float (&dn)[3]) {
+            if (last) {
 #pragma unroll
-              for (int m = 0; m < 9; ++m) qk1[m] = q[j + 1 < P ? j + 1 : j][m];
+              for (int c = 0; c < 3; ++c) {
+                xk1[c] = xt[c];
+                vk1[c] = vt[c];
+              }
+            } else if (j + 1 < P) {
+#pragma unroll
+              for (int c = 0; c < 3; ++c) {
+                xk1[c] = x[j + 1 < P ? j + 1 : j][c];
+                vk1[c] = v[j + 1 < P ? j + 1 : j][c];
+              }
             } else {
 #pragma unroll
-              for (int m = 0; m < 9; ++m) qk1[m] = s1[6 + m][tn];
+              for (int c = 0; c < 3; ++c) {
+                xk1[c] = s1[c][tn];
+                vk1[c] = s1[3 + c][tn];
+              }
             }
-            const bool next_last = (j + 1) % P == P - 1 && kk[j] + 1 == nn[j] - 1;
-            if (kCache && j == P - 1 && (P > 1 || next_last)) {
-              // FP32-bulk: the next element's rounded difference, from its thread
+            // the next lane's director and node difference; for a rod's last
+            // element they belong to the next rod (or to an idle lane: identity
+            // director, zero state) and only meet its zero Voronoi constants
+            // (FP32-bulk) or are not used (FP64)
+            {
+              if (j + 1 < P) {
 #pragma unroll
-              for (int c = 0; c < 3; ++c) dn[c] = s5[kCache ? c : 0][tn];
-            } else {
-              if (next_last) {
-                if (j + 1 < P) {
-#pragma unroll
-                  for (int c = 0; c < 3; ++c) xk2[c] = xt[c];
-                } else {
-#pragma unroll
-                  for (int c = 0; c < 3; ++c) xk2[c] = s1[kCache ? 0 : 15 + c][tn];
-                }
-              } else if (j + 2 < P) {
-#pragma unroll
-                for (int c = 0; c < 3; ++c) xk2[c] = x[j + 2 < P ? j + 2 : j][c];
-              } else if (j + 2 == P) {
-#pragma unroll
-                for (int c = 0; c < 3; ++c) xk2[c] = s1[c][tn];
-              } else if (P > 1) {
-#pragma unroll
-                for (int c = 0; c < 3; ++c) xk2[c] = s1[kCache ? 0 : 15 + c][tn];
+                for (int m = 0; m < 9; ++m) qk1[m] = q[j + 1 < P ? j + 1 : j][m];
               } else {
 #pragma unroll
-                for (int c = 0; c < 3; ++c) xk2[c] = s1[c][tn2];
+                for (int m = 0; m < 9; ++m) qk1[m] = s1[6 + m][tn];
               }
+              const bool next_last = (j + 1) % P == P - 1 && kk[j] + 1 == nn[j] - 1;
+              if (kCache && j == P - 1 && (P > 1 || next_last)) {
+                // FP32-bulk: the next element's rounded difference, from its thread
 #pragma unroll
-              for (int c = 0; c < 3; ++c) dn[c] = static_cast<float>(xk2[c] - xk1[c]);
+                for (int c = 0; c < 3; ++c) dn[c] = s5[kCache ? c : 0][tn];
+              } else {
+                if (next_last) {
+                  if (j + 1 < P) {
+#pragma unroll
+                    for (int c = 0; c < 3; ++c) xk2[c] = xt[c];
+                  } else {
+#pragma unroll
+                    for (int c = 0; c < 3; ++c) xk2[c] = s1[kCache ? 0 : 15 + c][tn];
+                  }
+                } else if (j + 2 < P) {
+#pragma unroll
+                  for (int c = 0; c < 3; ++c) xk2[c] = x[j + 2 < P ? j + 2 : j][c];
+                } else if (j + 2 == P) {
+#pragma unroll
+                  for (int c = 0; c < 3; ++c) xk2[c] = s1[c][tn];
+                } else if (P > 1) {
+#pragma unroll
+                  for (int c = 0; c < 3; ++c) xk2[c] = s1[kCache ? 0 : 15 + c][tn];
+                } else {
+#pragma unroll
+                  for (int c = 0; c < 3; ++c) xk2[c] = s1[c][tn2];
+                }
+#pragma unroll
+                for (int c = 0; c < 3; ++c) dn[c] = static_cast<float>(xk2[c] - xk1[c]);
+              }
             }
-          }
+          };
           ElemConst<R> K;
           if constexpr (kHold) {
             K = H;
@@ -1065,8 +1100,26 @@ namespace erod {
           R qr[9];
 #pragma unroll
           for (int m = 0; m < 9; ++m) qr[m] = static_cast<R>(q[j][m]);
-          element_forces<R>(x[j], xk1, xk2, dn, v[j], vk1, q[j], qr, qk1, w[j], has_vor, K, mid[j],
-                            kGeo ? geo[kGeo ? j : 0] : nullptr);
+          auto evaluate = [&](auto plain, step64::Range* range) __attribute__((always_inline)) {
+            double xk1[3], xk2[3] = {0, 0, 0}, vk1[3], qk1[9];
+            float dn[3] = {0.0f, 0.0f, 0.0f};
+            load_next(xk1, xk2, vk1, qk1, dn);
+            element_forces<R, plain.value>(x[j], xk1, xk2, dn, v[j], vk1, q[j], qr, qk1, w[j], has_vor, K, mid[j],
+                                           kGeo ? geo[kGeo ? j : 0] : nullptr, range);
+          };
+          if constexpr (kPlainFirst) {
+            // the plain form first; in a wave whose operands do not allow it all
+            // of it again, the next lanes' values read anew rather than kept in
+            // registers for this rare case
+            step64::Range range = consts;
+            evaluate(std::true_type(), &range);
+            if (step64::any(valid[j] && range.bad())) {
+              asm volatile("" ::: "memory");
+              evaluate(std::false_type(), nullptr);
+            }
+          } else {
+            evaluate(std::false_type(), nullptr);
+          }
         }
         // ---- exchange 2 -----------------------------------------------------------
 #pragma unroll
@@ -1231,12 +1284,12 @@ namespace erod {
 #pragma unroll
             for (int c = 0; c < 3; ++c) xt[c] = maddd<R>(ch, vt[c], xt[c]);
         }
-        if (kRuns && step + 1 == nsteps && rest > 0) {
+        if (kRuns && step + 1 == nsteps && __builtin_amdgcn_readfirstlane(rest) > 0) {
           // the next run of steps
 #pragma unroll
           for (int j = 0; j < P; ++j)
             if (lim[j] != kNoBudget) lim[j] = lim[j] > uint32_t(nsteps) ? lim[j] - uint32_t(nsteps) : 0u;
-          nsteps = split < rest ? split : rest;
+          nsteps = __builtin_amdgcn_readfirstlane(run < rest ? run : rest);
           rest -= nsteps;
           step = -1;
         }

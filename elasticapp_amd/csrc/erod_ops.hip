@@ -71,6 +71,7 @@ namespace erod {
     // mass of node k + 1
     struct SlotConst {
       double m, mn, im, gf, l0, gt, S[3], sigma0[3], J[3], iJ[3], D0, kappa0[3], B[3];
+      double il0, iD0;  // of step64::divisor
     };
 
     // bits of a slot's place: ghost node / element / Voronoi region, the
@@ -104,6 +105,8 @@ namespace erod {
       K.l0 = f.l0[ke];
       K.gt = f.gt[ke];
       K.D0 = f.D0[kv];
+      K.il0 = step64::divisor<true>(K.l0).r;
+      K.iD0 = step64::divisor<true>(K.D0).r;
 #pragma unroll
       for (int c = 0; c < 3; ++c) {
         K.S[c] = f.S[c * E + ke];
@@ -122,7 +125,10 @@ namespace erod {
     }
 
     // element_length = batch_norm(difference_kernel(position))
-    __device__ __forceinline__ double length(const double d[3]) { return sqrt(d[0] * d[0] + d[1] * d[1] + d[2] * d[2]); }
+    template <bool kPlain>
+    __device__ __forceinline__ double length(const double d[3]) {
+      return step64::root<kPlain>(d[0] * d[0] + d[1] * d[1] + d[2] * d[2]);
+    }
 
     // what slot k computes before it needs the terms of slot k - 1
     struct SlotTerms {
@@ -130,21 +136,31 @@ namespace erod {
       double qt[3], sigma[3], stress[3], c[3];    // Q t, strain, stress, Q^T n / e (0 at a ghost)
       double D, eps, kappa[3], couple[3], dv[3];  // Voronoi length, dilatation, curvature (0 at a ghost), couple, kappa x M
       double P[3], R[3];                          // M / eps^3, (kappa x M) D0 / eps^3
+      double jw[3];                               // J w / e
     };
 
-    __device__ __forceinline__ void slot_terms(const double x0[3], const double x1[3], const double x2[3],
-                                               const double q[9], const double qn[9], uint32_t place,
+    // (kPlain: divisions and roots without their special cases; returns bit 0 if
+    // an operand of the element's terms did not allow that, bit 1 if one of the
+    // Voronoi region's did not)
+    template <bool kPlain>
+    __device__ __forceinline__ uint32_t slot_terms(const double x0[3], const double x1[3], const double x2[3],
+                                               const double q[9], const double qn[9], const double w[3], uint32_t place,
                                                bool next_ghost_elem, const SlotConst& K, SlotTerms& o) {
+      using step64::Divisor;
+      using step64::divisor;
+      using step64::over;
       // update_spanwise_variables
       const double d[3] = {x1[0] - x0[0], x1[1] - x0[1], x1[2] - x0[2]};
       const double dn[3] = {x2[0] - x1[0], x2[1] - x1[1], x2[2] - x1[2]};
-      o.l = (place & kGhostElem) ? 1.0 : length(d);
-      const double ln = next_ghost_elem ? 1.0 : length(dn);
+      o.l = (place & kGhostElem) ? 1.0 : length<kPlain>(d);
+      const double ln = next_ghost_elem ? 1.0 : length<kPlain>(dn);
+      const Divisor byl = divisor<kPlain>(o.l), l0{K.l0, K.il0}, D0{K.D0, K.iD0};
 #pragma unroll
-      for (int c = 0; c < 3; ++c) o.t[c] = d[c] / o.l;
-      o.e = o.l / K.l0;
+      for (int c = 0; c < 3; ++c) o.t[c] = over<kPlain>(d[c], byl);
+      o.e = over<kPlain>(o.l, l0);
       o.D = 0.5 * (o.l + ln);
-      o.eps = o.D / K.D0;
+      o.eps = over<kPlain>(o.D, D0);
+      const Divisor bye = divisor<kPlain>(o.e);
       // update_shear_stretch_strain: sigma = (Q t) e - z; n = S % (sigma - sigma0)
 #pragma unroll
       for (int p = 0; p < 3; ++p) {
@@ -154,26 +170,47 @@ namespace erod {
       o.sigma[2] -= 1.0;
 #pragma unroll
       for (int p = 0; p < 3; ++p) o.stress[p] = K.S[p] * (o.sigma[p] - K.sigma0[p]);
-      // Q^T n / e with zeroed ghosts
+      // Q^T n / e with zeroed ghosts, and J w / e
+      double a[3], jw[3];
 #pragma unroll
       for (int j = 0; j < 3; ++j) {
-        const double a = q[j] * o.stress[0] + q[3 + j] * o.stress[1] + q[6 + j] * o.stress[2];
-        o.c[j] = (place & kGhostElem) ? 0.0 : a / o.e;
+        a[j] = q[j] * o.stress[0] + q[3 + j] * o.stress[1] + q[6 + j] * o.stress[2];
+        o.c[j] = (place & kGhostElem) ? 0.0 : over<kPlain>(a[j], bye);
+        jw[j] = K.J[j] * w[j];
+        o.jw[j] = over<kPlain>(jw[j], bye);
       }
       // curvature, couple, 1 / eps^3 and the terms of the torque sums
-      step64::curvature(q, qn, K.D0, o.kappa);
+      step64::curvature<kPlain>(q, qn, D0, o.kappa);
 #pragma unroll
       for (int c = 0; c < 3; ++c) {
         if (place & kGhostVor) o.kappa[c] = 0.0;
         o.couple[c] = K.B[c] * (o.kappa[c] - K.kappa0[c]);
       }
       cross(o.kappa, o.couple, o.dv);
-      const double ic = 1.0 / (o.eps * o.eps * o.eps), icd = ic * K.D0;
+      const double cube = o.eps * o.eps * o.eps;
+      const double ic = over<kPlain>(1.0, divisor<kPlain>(cube)), icd = ic * K.D0;
 #pragma unroll
       for (int c = 0; c < 3; ++c) {
         o.P[c] = o.couple[c] * ic;
         o.R[c] = o.dv[c] * icd;
       }
+      if constexpr (!kPlain) return 0u;
+      step64::Range elem, vor;
+      elem.divisor(o.l);
+      elem.divisor(o.e);
+      elem.divisor(K.l0);
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        elem.numerator(d[c]);
+        elem.numerator(a[c]);
+        elem.numerator(jw[c]);
+      }
+      elem.largest((((fabs(d[0]) + fabs(d[1])) + (fabs(d[2]) + fabs(a[0]))) + ((fabs(a[1]) + fabs(a[2])) + fabs(jw[0]))) +
+                   (fabs(jw[1]) + fabs(jw[2])));
+      vor.divisor(ln);
+      vor.divisor(K.D0);
+      vor.divisor(cube);
+      return ((place & kHasElem) && elem.bad() ? 1u : 0u) | ((place & kHasVor) && vor.bad() ? 2u : 0u);
     }
 
     // two_point_difference_kernel (BlazeCalculus.hpp:29-45) at one output,
@@ -197,13 +234,11 @@ namespace erod {
     // Lagrangian transport, unsteady dilatation, damping, added in this order
     __device__ __forceinline__ void slot_torque(const SlotTerms& s, const double Pm[3], const double Rm[3],
                                                 const double v0[3], const double v1[3], const double w[3],
-                                                uint32_t place, bool damped, const SlotConst& K, double jw[3],
-                                                double dvel[3], double tau[3]) {
+                                                uint32_t place, bool damped, const SlotConst& K, double dvel[3],
+                                                double tau[3]) {
       double shear[3], lag[3];
       cross(s.qt, s.stress, shear);
-#pragma unroll
-      for (int c = 0; c < 3; ++c) jw[c] = (K.J[c] * w[c]) / s.e;
-      cross(jw, w, lag);
+      cross(s.jw, w, lag);
 #pragma unroll
       for (int c = 0; c < 3; ++c) dvel[c] = v1[c] - v0[c];
       const double rate = (s.t[0] * dvel[0] + s.t[1] * dvel[1] + s.t[2] * dvel[2]) / (s.e * K.l0);
@@ -215,7 +250,7 @@ namespace erod {
         a += 0.5 * (first ? s.R[c] : (last ? Rm[c] : s.R[c] + Rm[c]));  // quadrature_kernel (BlazeCalculus.hpp:67-86)
         a += shear[c] * K.l0;
         a += lag[c];
-        a += jw[c] * rate;
+        a += s.jw[c] * rate;
         if (damped) a -= eg * w[c];
         tau[c] = a;
       }
@@ -278,11 +313,13 @@ namespace erod {
 #pragma unroll
       for (int m = 0; m < 9; ++m) {
         q[m] = f.q[m * E + ke];
-        qn[m] = f.q[m * E + kv + 1];
+        // (a ghost region's curvature is zero, and a missing one unused: its
+        // wave need not run the large-angle form for it)
+        qn[m] = f.q[m * E + ((place & kHasVor) && !(place & kGhostVor) ? k + 1 : ke)];
       }
       const double vol = f.vol[ke];
       const bool next_ghost = (place & kHasVor) && (is_ghost[k + 1] || is_ghost[k + 2]);
-      slot_terms(x[0], x[1], x[2], q, qn, place, next_ghost, K, o);
+      slot_terms<false>(x[0], x[1], x[2], q, qn, w, place, next_ghost, K, o);
 #pragma unroll
       for (int c = 0; c < 3; ++c) {
         s[c][tid] = o.c[c];
@@ -291,7 +328,7 @@ namespace erod {
       }
       __syncthreads();
       if (tid == 0 || !in) return;
-      double cm[3], Pm[3], Rm[3], fi[3], tau[3], jw[3], dvel[3];
+      double cm[3], Pm[3], Rm[3], fi[3], tau[3], dvel[3];
 #pragma unroll
       for (int c = 0; c < 3; ++c) {
         cm[c] = s[c][tid - 1];
@@ -305,7 +342,7 @@ namespace erod {
         f.f_ext[c * N + k] = 0.0;
       }
       if (place & kHasElem) {
-        slot_torque(o, Pm, Rm, v0, v1, w, place, damped, K, jw, dvel, tau);
+        slot_torque(o, Pm, Rm, v0, v1, w, place, damped, K, dvel, tau);
         f.l[k] = o.e * K.l0;  // (the reference leaves e l0 here, and eps D0 below)
         f.e[k] = o.e;
         f.r[k] = sqrt(M_1_PI * vol / o.l);  // update_dimension
@@ -316,7 +353,7 @@ namespace erod {
           f.stress[c * E + k] = o.stress[c];
           f.tau_int[c * E + k] = tau[c];
           f.tau_ext[c * E + k] = 0.0;
-          f.d1[c * E + k] = jw[c];
+          f.d1[c * E + k] = o.jw[c];
           f.d2[c * E + k] = dvel[c];
         }
       }
@@ -545,12 +582,21 @@ namespace erod {
       const bool whooks = __ballot(hooks != 0u) != 0ull;
       const bool environment = env.gravity || env.contact;
       const int n1 = tid + 1 < kThreads ? tid + 1 : tid, n2 = tid + 2 < kThreads ? tid + 2 : n1, p1 = tid > 0 ? tid - 1 : 0;
+      // Where a slot has no element, no Voronoi region, or no thread beside it
+      // to take one from, its terms are never used, and the curvature of a ghost
+      // region is zero: they get an unstrained element and their own director,
+      // so that their waves don't run the large-angle forms or, over values that
+      // are no numbers, the full ones.  Threads past the block's slots stand still.
+      const bool no_elem = !valid || !(place & kHasElem) || tid + 1 >= kThreads;
+      const bool no_vor = no_elem || !(place & kHasVor) || tid + 2 >= kThreads;
+      const bool own_q = no_vor || (place & kGhostVor);
+      const bool edge = step64::any(own_q);
+      const double dtk = valid ? dt : 0.0, ch = 0.5 * dtk;
       for (int step = 0; step < nsteps; ++step) {
-        const double ch = 0.5 * dt;
 #pragma unroll
         for (int c = 0; c < 3; ++c) x[c] += ch * v[c];
         step64::so3_update(q, w, ch);
-        t += ch;
+        t += 0.5 * dt;
         if (whooks && (hooks & 15u)) {
           const RodInfo& ri = rods[rod];
           for (int c = 0; c < 2; ++c) {
@@ -577,8 +623,23 @@ namespace erod {
         }
 #pragma unroll
         for (int m = 0; m < 9; ++m) qn[m] = s1[6 + m][n1];
+        if (edge) {
+#pragma unroll
+          for (int c = 0; c < 3; ++c) {
+            if (no_elem) x1[c] = x[c] + K.l0 * q[6 + c];
+            if (no_vor) x2[c] = x1[c] + (x1[c] - x[c]);
+          }
+#pragma unroll
+          for (int m = 0; m < 9; ++m)
+            if (own_q) qn[m] = q[m];
+        }
         SlotTerms o;
-        slot_terms(x, x1, x2, q, qn, place, next_ghost, K, o);
+        // (what lies past the last thread, and what a launch over several
+        // workgroups has already got wrong beside it, has no say)
+        const uint32_t bad = slot_terms<true>(x, x1, x2, q, qn, w, place, next_ghost, K, o);
+        const int sound = kThreads - 1 - (left > 0 ? step : 0);
+        if (step64::any(valid && (((bad & 1u) && tid < sound) || ((bad & 2u) && tid + 1 < sound))))
+          slot_terms<false>(x, x1, x2, q, qn, w, place, next_ghost, K, o);
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
           s3[c][tid] = o.c[c];
@@ -586,7 +647,7 @@ namespace erod {
           s3[6 + c][tid] = o.R[c];
         }
         __syncthreads();
-        double cm[3], Pm[3], Rm[3], fi[3], tau[3], jw[3], dvel[3], fe[3] = {0.0, 0.0, 0.0};
+        double cm[3], Pm[3], Rm[3], fi[3], tau[3], dvel[3], fe[3] = {0.0, 0.0, 0.0};
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
           cm[c] = s3[c][p1];
@@ -594,7 +655,7 @@ namespace erod {
           Rm[c] = s3[6 + c][p1];
         }
         slot_force(o.c, cm, v, place, damped, K, fi);
-        slot_torque(o, Pm, Rm, v, v1, w, place, damped, K, jw, dvel, tau);
+        slot_torque(o, Pm, Rm, v, v1, w, place, damped, K, dvel, tau);
         // forcing first, then environments
         if (whooks && (hooks & 16u)) {
           const RodInfo& ri = rods[rod];
@@ -604,8 +665,8 @@ namespace erod {
         if (environment) add_environment(env, K.m, x, v, place & kGhostNode, fe);
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
-          v[c] += dt * ((fi[c] + fe[c]) * K.im);
-          w[c] += dt * ((K.iJ[c] * (tau[c] + 0.0)) * o.e);  // (the external torque is zero)
+          v[c] += dtk * ((fi[c] + fe[c]) * K.im);
+          w[c] += dtk * ((K.iJ[c] * (tau[c] + 0.0)) * o.e);  // (the external torque is zero)
         }
         if (whooks) {
           if (hooks & 3u)
@@ -613,7 +674,7 @@ namespace erod {
           if (hooks & 12u)
             for (int c = 0; c < 3; ++c) w[c] = 0.0;
         }
-        t += ch;
+        t += 0.5 * dt;
 #pragma unroll
         for (int c = 0; c < 3; ++c) x[c] += ch * v[c];
         step64::so3_update(q, w, ch);

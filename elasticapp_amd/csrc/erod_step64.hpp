@@ -9,6 +9,75 @@
 namespace erod {
   namespace step64 {
 
+    // ---- division and square root without their special cases -------------------
+    //
+    // An FP64 division is 11 instructions: the divisor's reciprocal by Newton's
+    // iteration from v_rcp_f64, the quotient by it, one correction from the
+    // exact remainder (Markstein), and four more that scale extreme operands
+    // and patch special results.  Where no operand is extreme the scaling is by
+    // one, and the same steps without it give the same bits (a zero quotient
+    // may lose its sign); several numerators over one divisor then share the
+    // iteration, and a constant divisor's can be made once.  A square root is
+    // 18 instructions of which 10 remain.  kPlain code below takes these forms
+    // and notes in a Range whether every operand allowed them; a wave in which
+    // one did not computes the terms again with the full forms.  The FP64 step is
+    // bound by VALU issue: 1,190 -> 970 instructions of the fused one, 1,024 rods
+    // of 64 elements 1.65 -> 1.50 ms per 500 steps, 2,048 ragged rods 8.4 -> 7.1 ms
+    // per 300, op-by-op steps of 248,188 elements 14.4 -> 13.5 us each.
+
+    // operands met so far: bad if a divisor or radicand lies outside 2^-100 ...
+    // 2^100, a numerator other than zero below 2^-800, or one above 2^600
+    struct Range {
+      uint32_t least = 0xffffffffu;  // smallest (high word << 1) - 1; a zero's is the largest
+      bool out = false;
+
+      __device__ __forceinline__ static uint32_t high(double v) { return static_cast<uint32_t>(__double2hiint(v)); }
+      __device__ __forceinline__ void divisor(double d) {
+        out |= high(d) - ((1023u - 100u) << 20) >= (200u << 20);  // (a negative one, an infinity or a NaN too)
+      }
+      // a numerator known not to be large
+      __device__ __forceinline__ void numerator(double n) { least = min(least, (high(n) << 1) - 1u); }
+      // the largest magnitude of numerators that may be
+      __device__ __forceinline__ void largest(double a) { out |= !(a < 0x1p600); }
+      __device__ __forceinline__ bool bad() const { return out || least < ((1023u - 800u) << 21); }
+    };
+
+    // a divisor with its reciprocal
+    struct Divisor {
+      double d, r;
+    };
+
+    template <bool kPlain>
+    __device__ __forceinline__ Divisor divisor(double d) {
+      if constexpr (!kPlain) return {d, 0.0};
+      double r = __builtin_amdgcn_rcp(d);
+      r = __builtin_fma(r, __builtin_fma(-d, r, 1.0), r);
+      r = __builtin_fma(r, __builtin_fma(-d, r, 1.0), r);
+      return {d, r};
+    }
+
+    template <bool kPlain>
+    __device__ __forceinline__ double over(double n, const Divisor& by) {
+      if constexpr (!kPlain) return n / by.d;
+      const double q = n * by.r;
+      return __builtin_fma(__builtin_fma(-by.d, q, n), by.r, q);
+    }
+
+    template <bool kPlain>
+    __device__ __forceinline__ double root(double x) {
+      if constexpr (!kPlain) return sqrt(x);
+      const double y = __builtin_amdgcn_rsq(x);
+      double g = x * y, h = 0.5 * y;
+      const double e = __builtin_fma(-h, g, 0.5);
+      g = __builtin_fma(g, e, g);
+      h = __builtin_fma(h, e, h);
+      g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
+      return __builtin_fma(__builtin_fma(-g, g, x), h, g);
+    }
+
+    // whether any lane of the wave has `b`
+    __device__ __forceinline__ bool any(bool b) { return __ballot(b) != 0ull; }
+
     // Q <- exp(-[u]x) Q with u = c w: SO3AddAssign<scalar>
     // (SO3PrimitiveAddAssign/Scalar.hpp:25-96)
     __device__ __forceinline__ void so3_update(double q[9], const double w[3], double c) {
@@ -18,9 +87,22 @@ namespace erod {
       math::sincos(theta, &beta, &c_alpha);
       const double alpha = 1.0 - c_alpha;
       const double den = theta + 1e-14;
-      u0 /= den;
-      u1 /= den;
-      u2 /= den;
+      // (|u| <= theta: no numerator is large when den is not)
+      Range g;
+      g.divisor(den);
+      g.numerator(u0);
+      g.numerator(u1);
+      g.numerator(u2);
+      if (any(g.bad())) {
+        u0 /= den;
+        u1 /= den;
+        u2 /= den;
+      } else {
+        const Divisor by = divisor<true>(den);
+        u0 = over<true>(u0, by);
+        u1 = over<true>(u1, by);
+        u2 = over<true>(u2, by);
+      }
 #pragma unroll
       for (int j = 0; j < 3; ++j) {
         const double a = q[j], b = q[3 + j], cc = q[6 + j];
@@ -33,11 +115,13 @@ namespace erod {
 
     // curvature between neighbouring directors: InvRotateDivideOp<scalar>
     // (InvRotateDivide/Scalar.hpp:26-110)
-    __device__ __forceinline__ void curvature(const double qc[9], const double qn[9], double D0, double kap[3]) {
+    template <bool kPlain>
+    __device__ __forceinline__ void curvature(const double qc[9], const double qn[9], const Divisor& D0, double kap[3]) {
       const double tr = qc[0] * qn[0] + qc[1] * qn[1] + qc[2] * qn[2] + qc[3] * qn[3] + qc[4] * qn[4] +
                         qc[5] * qn[5] + qc[6] * qn[6] + qc[7] * qn[7] + qc[8] * qn[8];
       const double theta = math::acos(0.5 * tr - (0.5 + 1e-10));
-      const double st = 0.5 * theta / math::sin(theta + 1e-14) / D0;
+      // (theta / 2 sin(theta) is zero, NaN or between 1/2 and 2^50)
+      const double st = over<kPlain>(0.5 * theta / math::sin(theta + 1e-14), D0);
       kap[0] = st * (-qc[3] * qn[6] - qc[4] * qn[7] - qc[5] * qn[8] + qc[6] * qn[3] + qc[7] * qn[4] + qc[8] * qn[5]);
       kap[1] = st * (qc[0] * qn[6] + qc[1] * qn[7] + qc[2] * qn[8] - qc[6] * qn[0] - qc[7] * qn[1] - qc[8] * qn[2]);
       kap[2] = st * (-qc[0] * qn[3] - qc[1] * qn[4] - qc[2] * qn[5] + qc[3] * qn[0] + qc[4] * qn[1] + qc[5] * qn[2]);
