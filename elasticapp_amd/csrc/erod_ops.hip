@@ -592,10 +592,13 @@ namespace erod {
       const bool own_q = no_vor || (place & kGhostVor);
       const bool edge = step64::any(own_q);
       const double dtk = valid ? dt : 0.0, ch = 0.5 * dtk;
+      // (the half step that closes a step turns by the rotation of the one that
+      // opens the next)
+      step64::Rotation turn = step64::rotation(w, ch);
       for (int step = 0; step < nsteps; ++step) {
 #pragma unroll
         for (int c = 0; c < 3; ++c) x[c] += ch * v[c];
-        step64::so3_update(q, w, ch);
+        step64::rotate(q, turn);
         t += 0.5 * dt;
         if (whooks && (hooks & 15u)) {
           const RodInfo& ri = rods[rod];
@@ -677,7 +680,8 @@ namespace erod {
         t += 0.5 * dt;
 #pragma unroll
         for (int c = 0; c < 3; ++c) x[c] += ch * v[c];
-        step64::so3_update(q, w, ch);
+        turn = step64::rotation(w, ch);
+        step64::rotate(q, turn);
       }
       if (!valid || tid < left || tid >= left + own) return;
 #pragma unroll

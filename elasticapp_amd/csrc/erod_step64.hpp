@@ -78,14 +78,17 @@ namespace erod {
     // whether any lane of the wave has `b`
     __device__ __forceinline__ bool any(bool b) { return __ballot(b) != 0ull; }
 
-    // Q <- exp(-[u]x) Q with u = c w: SO3AddAssign<scalar>
-    // (SO3PrimitiveAddAssign/Scalar.hpp:25-96)
-    __device__ __forceinline__ void so3_update(double q[9], const double w[3], double c) {
+    // the rotation exp(-[u]x), u = c w: its axis and the sine and cosine of
+    // its angle
+    struct Rotation {
+      double u[3], beta, c_alpha;
+    };
+
+    __device__ __forceinline__ Rotation rotation(const double w[3], double c) {
+      Rotation o;
       double u0 = c * w[0], u1 = c * w[1], u2 = c * w[2];
       const double theta = sqrt(u0 * u0 + u1 * u1 + u2 * u2);
-      double beta, c_alpha;
-      math::sincos(theta, &beta, &c_alpha);
-      const double alpha = 1.0 - c_alpha;
+      math::sincos(theta, &o.beta, &o.c_alpha);
       const double den = theta + 1e-14;
       // (|u| <= theta: no numerator is large when den is not)
       Range g;
@@ -103,6 +106,16 @@ namespace erod {
         u1 = over<true>(u1, by);
         u2 = over<true>(u2, by);
       }
+      o.u[0] = u0;
+      o.u[1] = u1;
+      o.u[2] = u2;
+      return o;
+    }
+
+    // Q <- exp(-[u]x) Q
+    __device__ __forceinline__ void rotate(double q[9], const Rotation& o) {
+      const double u0 = o.u[0], u1 = o.u[1], u2 = o.u[2], beta = o.beta, c_alpha = o.c_alpha;
+      const double alpha = 1.0 - c_alpha;
 #pragma unroll
       for (int j = 0; j < 3; ++j) {
         const double a = q[j], b = q[3 + j], cc = q[6 + j];
@@ -111,6 +124,12 @@ namespace erod {
         q[3 + j] = c_alpha * b + alpha * u1 * com + beta * (cc * u0 - a * u2);
         q[6 + j] = c_alpha * cc + alpha * u2 * com + beta * (a * u1 - b * u0);
       }
+    }
+
+    // Q <- exp(-[u]x) Q with u = c w: SO3AddAssign<scalar>
+    // (SO3PrimitiveAddAssign/Scalar.hpp:25-96)
+    __device__ __forceinline__ void so3_update(double q[9], const double w[3], double c) {
+      rotate(q, rotation(w, c));
     }
 
     // curvature between neighbouring directors: InvRotateDivideOp<scalar>
