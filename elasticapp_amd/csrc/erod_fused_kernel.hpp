@@ -125,6 +125,25 @@ namespace erod {
       o[2] = madd(a[0], b[1], -(a[1] * b[0]));
     }
 
+    // the next and the previous lane's value; the wave's last, its first lane
+    // gets zero.  Every lane of the wave has to be on.  (wave_shl:1, wave_shr:1)
+    template <int kCtrl>
+    __device__ __forceinline__ int lane_move(int v) {
+      return __builtin_amdgcn_update_dpp(0, v, kCtrl, 0xf, 0xf, true);
+    }
+    template <int kCtrl>
+    __device__ __forceinline__ float lane_move(float v) {
+      return __int_as_float(lane_move<kCtrl>(__float_as_int(v)));
+    }
+    template <int kCtrl>
+    __device__ __forceinline__ double lane_move(double v) {
+      return __hiloint2double(lane_move<kCtrl>(__double2hiint(v)), lane_move<kCtrl>(__double2loint(v)));
+    }
+    template <typename T>
+    __device__ __forceinline__ T lane_next(T v) { return lane_move<0x130>(v); }
+    template <typename T>
+    __device__ __forceinline__ T lane_prev(T v) { return lane_move<0x138>(v); }
+
     using step64::ramp_value;
 
     // ---- director update Q <- exp(-[u]x) Q, u = c w, in FP64 ----------------------
@@ -199,14 +218,15 @@ namespace erod {
       return __builtin_fma(-c[2], d[2], s);
     }
 
-    __device__ __forceinline__ void curvature32(const double qc[9], const double qn[9], float iD0, float kap[3]) {
+    __device__ __forceinline__ void curvature32(const double qc[9], const double qn[9], float iD0, float kap[3],
+                                                bool unused = false) {
       const double tr = dot3_fma(qc, qn) + dot3_fma(qc + 3, qn + 3) + dot3_fma(qc + 6, qn + 6);
       // rows: d1 = q[0..2], d2 = q[3..5], d3 = q[6..8]
       const double s0 = skew3_fma(qc + 6, qn + 3, qc + 3, qn + 6);
       const double s1 = skew3_fma(qc + 0, qn + 6, qc + 6, qn + 0);
       const double s2 = skew3_fma(qc + 3, qn + 0, qc + 0, qn + 3);
       float a = static_cast<float>((3.0 - tr) * 0.25) + 5e-11f;
-      a = fminf(fmaxf(a, 0.0f), 1.0f);
+      a = unused ? 0.0f : fminf(fmaxf(a, 0.0f), 1.0f);
       // st = (theta / 2) / sin(theta) / D0 with a = sin^2(theta / 2):
       // theta / (2 sin theta) = g(a) / 2, g(a) = asin(sqrt a) / (sqrt(a) sqrt(1 - a))
       //                      = sum_n 4^n (n!)^2 / (2n + 1)! a^n = 1 + 2a/3 + 8a^2/15 + 16a^3/35 + 128a^4/315 + ...
@@ -289,7 +309,9 @@ namespace erod {
     // (the FP64 state for R = double, its FP32 copy for R = float).  kPlain
     // (FP64): divisions and roots without their special cases, `range` noting
     // whether the operands allowed that.
-    template <typename R, bool kPlain = false>
+    // kWave: the next element is the next lane's, from which its length comes;
+    // every lane of the wave is here.
+    template <typename R, bool kPlain = false, bool kWave = false>
     __device__ __forceinline__ void element_forces(const double xk[3], const double xk1[3], const double xk2[3],
                                                    const float dn[3], const double vk[3], const double vk1[3],
                                                    const double qk[9], const R qr[9], const double qk1[9],
@@ -408,9 +430,11 @@ namespace erod {
       // reference's acos(tr / 2 - 1/2 - 1e-10), which is not defined for a
       // relative rotation of pi (a rod's last director against an idle lane's
       // identity), so it branches.
+      R l1 = kWave && sizeof(R) == 8 ? lane_next(l) : R(0);
       if (sizeof(R) == 4 || has_vor) {
-        R l1;
-        if constexpr (sizeof(R) == 8) {
+        if constexpr (sizeof(R) == 8 && kWave) {
+          if constexpr (kPlain) range->divisor(l1);
+        } else if constexpr (sizeof(R) == 8) {
           const double f0 = xk2[0] - xk1[0], f1 = xk2[1] - xk1[1], f2 = xk2[2] - xk1[2];
           l1 = step64::root<kPlain>(f0 * f0 + f1 * f1 + f2 * f2);
           if constexpr (kPlain) range->divisor(l1);
@@ -426,7 +450,7 @@ namespace erod {
           step64::curvature<kPlain>(qk, qk1, D0, kap);
         } else {
           eps = D * K.iD0;
-          curvature32(qk, qk1, K.iD0, kap);
+          curvature32(qk, qk1, K.iD0, kap, kWave && !has_vor);
         }
         R M[3];
 #pragma unroll
@@ -577,6 +601,15 @@ namespace erod {
       // is no room: FP64 reads them every step, FP32-bulk from the table.
       constexpr bool kHold = P == 1;
       constexpr bool kPlainFirst = kHold && !kCache;
+      // A tile of one wave, one element per thread: neighbours' values move
+      // between lanes by DPP instead of through LDS, whose 31 accesses a step
+      // (216 of its cycles per wave, shared by the waves of a CU) and their
+      // latency were a third of a step's time with one wave per SIMD; the next
+      // element's length comes along instead of being formed again.  1,024
+      // rods of 64 elements, us a step: FP32-bulk 1.44 -> 1.14 (VALU
+      // instructions 364 -> 384, cycles 3,030 -> 2,200), FP64 3.05 -> 2.75 (885
+      // -> 916, 6,270 -> 5,340)
+      constexpr bool kWave = P == 1 && NT == 64;
       // FP32-bulk: the closing half step of one step and the opening half step
       // of the next (same v and w) are taken as one update of dt within a launch
       constexpr bool kMerge = sizeof(R) == 4;
@@ -961,9 +994,9 @@ namespace erod {
         // FP32-bulk with P > 1: per element, the FP32-rounded node difference
         // and its length (geo[j] = {d, |d|, next element's |d|}), the first
         // element's before the exchange, which publishes both
-        constexpr bool kGeo = kCache && P > 1;
+        constexpr bool kGeo = kCache && (P > 1 || kWave);
         float geo[kGeo ? P : 1][5];
-        {
+        if constexpr (!kWave) {
           const bool last0 = P == 1 && valid[0] && (kk[0] == nn[0] - 1);
 #pragma unroll
           for (int c = 0; c < 3; ++c) {
@@ -982,11 +1015,11 @@ namespace erod {
           }
 #pragma unroll
           for (int m = 0; m < 9; ++m) s1[6 + m][tid] = q[0][m];
+          __syncthreads();
         }
-        __syncthreads();
         const int tn = tid + 1 < NT ? tid + 1 : tid;
         const int tn2 = tid + 2 < NT ? tid + 2 : tn;
-        if constexpr (kGeo) {
+        if constexpr (kGeo && !kWave) {
 #pragma unroll
           for (int j = 1; j < P; ++j) {
             const bool lastj = j == P - 1 && kk[j] == nn[j] - 1;
@@ -1010,7 +1043,7 @@ namespace erod {
         Mid<R> mid[P];
 #pragma unroll
         for (int j = 0; j < P; ++j) {
-          if (kEnv == 2 && !valid[j]) {
+          if (kEnv == 2 && !kWave && !valid[j]) {
             // (the tilted plane's kernel keeps the branch: without it, the
             // compiler's schedule for it needs more than 256 registers)
 #pragma unroll
@@ -1020,9 +1053,26 @@ namespace erod {
             continue;
           }
           const bool last = j == P - 1 && kk[j] == nn[j] - 1;
-          const bool has_vor = !last && !pad[j];
+          const bool has_vor = !last && !pad[j] && (!kWave || tid + 1 < NT);
           // the values of the next lanes
           auto load_next = [&](double (&xk1)[3], double (&xk2)[3], double (&vk1)[3], double (&qk1)[9], float (&dn)[3]) {
+            if constexpr (kWave) {
+#pragma unroll
+              for (int c = 0; c < 3; ++c) {
+                const double xn = lane_next(x[j][c]), vn = lane_next(v[j][c]);
+                xk1[c] = last ? xt[c] : xn;
+                vk1[c] = last ? vt[c] : vn;
+              }
+#pragma unroll
+              for (int m = 0; m < 9; ++m) qk1[m] = lane_next(q[j][m]);
+              if constexpr (kCache) {
+#pragma unroll
+                for (int c = 0; c < 3; ++c) geo[0][c] = static_cast<float>(xk1[c] - x[j][c]);
+                geo[0][3] = len32(geo[0][0], geo[0][1], geo[0][2]);
+                geo[0][4] = lane_next(geo[0][3]);
+              }
+              return;
+            }
             if (last) {
 #pragma unroll
               for (int c = 0; c < 3; ++c) {
@@ -1113,7 +1163,7 @@ namespace erod {
             double xk1[3], xk2[3] = {0, 0, 0}, vk1[3], qk1[9];
             float dn[3] = {0.0f, 0.0f, 0.0f};
             load_next(xk1, xk2, vk1, qk1, dn);
-            element_forces<R, plain.value>(x[j], xk1, xk2, dn, v[j], vk1, q[j], qr, qk1, w[j], has_vor, K, mid[j],
+            element_forces<R, plain.value, kWave>(x[j], xk1, xk2, dn, v[j], vk1, q[j], qr, qk1, w[j], has_vor, K, mid[j],
                                            kGeo ? geo[kGeo ? j : 0] : nullptr, range);
           };
           if constexpr (kPlainFirst) {
@@ -1131,13 +1181,23 @@ namespace erod {
           }
         }
         // ---- exchange 2 -----------------------------------------------------------
+        R before[kWave ? 9 : 1];
+        if constexpr (kWave) {
 #pragma unroll
-        for (int c = 0; c < 3; ++c) {
-          s3[c][tid + 1] = mid[P - 1].c[c];
-          s3[3 + c][tid + 1] = mid[P - 1].P[c];
-          s3[6 + c][tid + 1] = mid[P - 1].Rv[c];
+          for (int c = 0; c < 3; ++c) {
+            before[kWave ? c : 0] = lane_prev(mid[0].c[c]);
+            before[kWave ? 3 + c : 0] = lane_prev(mid[0].P[c]);
+            before[kWave ? 6 + c : 0] = lane_prev(mid[0].Rv[c]);
+          }
+        } else {
+#pragma unroll
+          for (int c = 0; c < 3; ++c) {
+            s3[c][tid + 1] = mid[P - 1].c[c];
+            s3[3 + c][tid + 1] = mid[P - 1].P[c];
+            s3[6 + c][tid + 1] = mid[P - 1].Rv[c];
+          }
+          __syncthreads();
         }
-        __syncthreads();
 #pragma unroll
         for (int j = 0; j < P; ++j) {
           if (!live[j]) continue;
@@ -1150,9 +1210,15 @@ namespace erod {
           R cm[3], Pm[3], Rm[3];
 #pragma unroll
           for (int c = 0; c < 3; ++c) {
-            cm[c] = j > 0 ? mid[j > 0 ? j - 1 : 0].c[c] : s3[c][tid];
-            Pm[c] = j > 0 ? mid[j > 0 ? j - 1 : 0].P[c] : s3[3 + c][tid];
-            Rm[c] = j > 0 ? mid[j > 0 ? j - 1 : 0].Rv[c] : s3[6 + c][tid];
+            if constexpr (kWave) {
+              cm[c] = before[kWave ? c : 0];
+              Pm[c] = before[kWave ? 3 + c : 0];
+              Rm[c] = before[kWave ? 6 + c : 0];
+            } else {
+              cm[c] = j > 0 ? mid[j > 0 ? j - 1 : 0].c[c] : s3[c][tid];
+              Pm[c] = j > 0 ? mid[j > 0 ? j - 1 : 0].P[c] : s3[3 + c][tid];
+              Rm[c] = j > 0 ? mid[j > 0 ? j - 1 : 0].Rv[c] : s3[6 + c][tid];
+            }
             cm[c] = first ? R(0) : cm[c];
           }
           const uint64_t s = slot[j];
