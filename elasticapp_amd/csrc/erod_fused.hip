@@ -134,7 +134,8 @@ namespace erod {
     return b->plan.lanes_per_tile == 0 && b->plan.elements_per_thread == 0 && b->plan.tuned_shape < 0;
   }
 
-  constexpr int kShape256 = 2, kShape512 = 3;  // one element per thread
+  constexpr int kShape256 = 2, kShape512 = 3;      // one element per thread
+  constexpr int kShape128x2 = 8, kShape512x2 = 4;  // two
 
   // Default shape without measurement: the smallest capacity that holds the
   // longest rod; one element per thread up to 256 lanes, two elements per
@@ -147,10 +148,16 @@ namespace erod {
   // which is shorter at one element per thread (600 such rods: 2.40 against
   // 2.65; 61 rods of up to 301: 2.15 against 2.67); fused FP64 has no registers
   // for two (17.5 against 21.0 for 2,400 rods, 5.7 against 7.1 for 61).
+  // FP32-bulk batches of shorter rods take two elements per thread too once
+  // they fill the SIMDs, where fewer instructions per element count: rods of up
+  // to 128 elements in 128-lane tiles of one wave (8,192 rods of 128: 9.8 us a
+  // step against 13.9; 1,024: 1.87 and 1.93; 512: 1.81 and 1.62; rods of 64:
+  // 8,192 5.25 and 6.28, 3,072 2.84 and 3.01, 2,048 1.90 and 1.69), rods of up
+  // to 256 in 512-lane ones (4,096 of 256: 11.2 and 13.3; 512: 2.41 and 2.02).
   // A shape the autotuner chose is taken again while it stays feasible (a
   // replan after rods changed length keeps it, with its second group).
   static int default_shape(const erod_batch* b, int precision) {
-    static const int pref[] = {0, 1, 2, 4, 5, 3, 7, 6};
+    static const int pref[] = {0, 1, 2, 4, 5, 3, 7, 6, 8};
     if (b->plan.tuned_shape >= 0 && shape_feasible(b, b->plan.tuned_shape)) return b->plan.tuned_shape;
     uint64_t maxn = 0, lanes = 0;
     for (uint64_t r = 0; r < b->n_rods; ++r)
@@ -161,11 +168,16 @@ namespace erod {
     for (int si : pref)
       if (uint64_t(fused_shape_lanes(si)) >= maxn && shape_feasible(b, si)) {
         const bool two = fused_shape_lanes(si) == 512 && fused_shape_epl(si) == 2;
+        if (precision != EROD_FP64 && shapes_free(b)) {
+          const uint64_t cus = uint64_t(b->cus);
+          if (maxn <= 128 && lanes > (maxn <= 64 ? 640 : 512) * cus && shape_feasible(b, kShape128x2)) return kShape128x2;
+          if (maxn > 128 && maxn <= 256 && lanes > 1024 * cus && shape_feasible(b, kShape512x2)) return kShape512x2;
+        }
         if (two && shape_feasible(b, kShape512) && (precision == EROD_FP64 || lanes <= 512 * uint64_t(b->cus))) return kShape512;
         return si;
       }
     // longer rods than any tile: the largest tiles, the longer rods in pieces
-    for (int si : {5, 4, 3, 2, 1, 0, 7, 6})
+    for (int si : {5, 4, 3, 2, 1, 0, 7, 6, 8})
       if (shape_feasible(b, si)) return si;
     return -1;
   }
@@ -181,7 +193,7 @@ namespace erod {
   // / 7.0 and 22.8 / 13.7 / 13.1.
   static int piece_shape(const erod_batch* b, int main_shape, int precision) {
     if (b->plan.seg_lanes > 0) {
-      for (int si : {0, 1, 2, 4, 5, 3, 7, 6})  // the default order of preference
+      for (int si : {0, 1, 2, 4, 5, 3, 7, 6, 8})  // the default order of preference
         if (fused_shape_lanes(si) == b->plan.seg_lanes && (b->plan.seg_epl <= 0 || fused_shape_epl(si) == b->plan.seg_epl))
           return si;
       return -2;
@@ -361,7 +373,7 @@ namespace erod {
   // the shape a requested second group uses, or -1 (none requested)
   static int split_shape(const erod_batch* b) {
     if (b->plan.split_lanes <= 0) return -1;
-    for (int si : {0, 1, 2, 4, 5, 3, 7, 6})  // the default order of preference
+    for (int si : {0, 1, 2, 4, 5, 3, 7, 6, 8})  // the default order of preference
       if (fused::kShapes[si].P * fused::kShapes[si].NT == b->plan.split_lanes &&
           (b->plan.split_epl <= 0 || fused::kShapes[si].P == b->plan.split_epl))
         return si;
@@ -612,10 +624,13 @@ namespace erod {
     // pieces of the requested shape, or of the main one
     auto tuned_pieces = [&](int si) { return b->plan.seg_lanes > 0 ? piece_shape(b, si, precision) : si; };
     b->plan.kept.valid = false;
+    // (fused FP64 has no registers for two elements: 47 us a step on 8,192 rods
+    // of 128 elements, 29 at one)
+    auto candidate = [&](int si) { return si != kShape128x2 || precision != EROD_FP64; };
     int best = -1;
     double best_t = 0.0;
     for (int si = 0; si < fused::kNShapes && rc == EROD_OK; ++si) {
-      if (!shape_feasible(b, si)) continue;
+      if (!shape_feasible(b, si) || !candidate(si)) continue;
       if ((rc = plan_tiles(b, si, tuned_pieces(si), precision))) break;
       if ((rc = fused_launch(b, precision, trial_steps, false))) break;  // warm
       if ((rc = fused_launch(b, precision, trial_steps, true))) break;
@@ -633,7 +648,7 @@ namespace erod {
     if (rc == EROD_OK && best >= 0 && g.split_lanes == 0) {
       const int cap = fused_shape_lanes(best);
       for (int s2 = 0; s2 < fused::kNShapes && rc == EROD_OK; ++s2) {
-        if (fused_shape_lanes(s2) >= cap) continue;
+        if (fused_shape_lanes(s2) >= cap || !candidate(s2)) continue;
         b->plan.split_lanes = fused_shape_lanes(s2);
         b->plan.split_epl = fused_shape_epl(s2);
         const int prc = plan_tiles(b, best, tuned_pieces(best), precision);

@@ -601,15 +601,19 @@ namespace erod {
       // is no room: FP64 reads them every step, FP32-bulk from the table.
       constexpr bool kHold = P == 1;
       constexpr bool kPlainFirst = kHold && !kCache;
-      // A tile of one wave, one element per thread: neighbours' values move
-      // between lanes by DPP instead of through LDS, whose 31 accesses a step
-      // (216 of its cycles per wave, shared by the waves of a CU) and their
-      // latency were a third of a step's time with one wave per SIMD; the next
-      // element's length comes along instead of being formed again.  1,024
-      // rods of 64 elements, us a step: FP32-bulk 1.44 -> 1.14 (VALU
-      // instructions 364 -> 384, cycles 3,030 -> 2,200), FP64 3.05 -> 2.75 (885
-      // -> 916, 6,270 -> 5,340)
-      constexpr bool kWave = P == 1 && NT == 64;
+      // A tile of one wave: neighbours' values move between lanes by DPP instead
+      // of through LDS, whose 31 accesses a step (216 of its cycles per wave,
+      // shared by the waves of a CU) and their latency were a third of a step's
+      // time with one wave per SIMD; the next element's length comes along
+      // instead of being formed again.  1,024 rods of 64 elements, us a step:
+      // FP32-bulk 1.44 -> 1.14 (VALU instructions 364 -> 384, cycles 3,030 ->
+      // 2,200), FP64 3.05 -> 2.75 (885 -> 916, 6,270 -> 5,340).  With two
+      // elements per thread the moves are shared by both: 8,192 rods of 128 with
+      // contact 11.0, against 12.4 in tiles of four waves through LDS and 14.9
+      // at one element per thread.  (Tiles of several waves at one element per
+      // thread, with only the waves' edge lanes through LDS, were 0 to 5% slower
+      // than with all of them: the barrier stays, and the moves come on top.)
+      constexpr bool kWave = NT == 64 && (P == 1 || kCache);
       // FP32-bulk: the closing half step of one step and the opening half step
       // of the next (same v and w) are taken as one update of dt within a launch
       constexpr bool kMerge = sizeof(R) == 4;
@@ -996,6 +1000,16 @@ namespace erod {
         // element's before the exchange, which publishes both
         constexpr bool kGeo = kCache && (P > 1 || kWave);
         float geo[kGeo ? P : 1][5];
+        double xnext[kWave ? 3 : 1];
+        if constexpr (kWave) {
+#pragma unroll
+          for (int c = 0; c < 3; ++c) xnext[kWave ? c : 0] = lane_next(x[0][c]);
+        }
+        if constexpr (kWave && P > 1) {
+#pragma unroll
+          for (int c = 0; c < 3; ++c) geo[0][c] = static_cast<float>(x[P > 1 ? 1 : 0][c] - x[0][c]);
+          geo[0][3] = len32(geo[0][0], geo[0][1], geo[0][2]);
+        }
         if constexpr (!kWave) {
           const bool last0 = P == 1 && valid[0] && (kk[0] == nn[0] - 1);
 #pragma unroll
@@ -1019,19 +1033,19 @@ namespace erod {
         }
         const int tn = tid + 1 < NT ? tid + 1 : tid;
         const int tn2 = tid + 2 < NT ? tid + 2 : tn;
-        if constexpr (kGeo && !kWave) {
+        if constexpr (kGeo && P > 1) {
 #pragma unroll
           for (int j = 1; j < P; ++j) {
             const bool lastj = j == P - 1 && kk[j] == nn[j] - 1;
 #pragma unroll
             for (int c = 0; c < 3; ++c) {
-              const double xn = lastj ? xt[c] : (j + 1 < P ? x[j + 1 < P ? j + 1 : j][c] : s1[c][tn]);
+              const double xn = lastj ? xt[c] : (j + 1 < P ? x[j + 1 < P ? j + 1 : j][c] : (kWave ? xnext[kWave ? c : 0] : s1[c][tn]));
               geo[kGeo ? j : 0][c] = static_cast<float>(xn - x[j][c]);
             }
             geo[kGeo ? j : 0][3] = len32(geo[kGeo ? j : 0][0], geo[kGeo ? j : 0][1], geo[kGeo ? j : 0][2]);
           }
 #pragma unroll
-          for (int j = 0; j < P; ++j) geo[kGeo ? j : 0][4] = j + 1 < P ? geo[kGeo ? (j + 1 < P ? j + 1 : j) : 0][3] : s5[kCache ? 3 : 0][tn];
+          for (int j = 0; j < P; ++j) geo[kGeo ? j : 0][4] = j + 1 < P ? geo[kGeo ? (j + 1 < P ? j + 1 : j) : 0][3] : (kWave ? lane_next(geo[0][3]) : s5[kCache ? 3 : 0][tn]);
         }
         // Idle lanes (past the tile's last entry) and pad lanes compute on
         // their stand-in state and constants too.  A tile's entries end on a
@@ -1053,14 +1067,14 @@ namespace erod {
             continue;
           }
           const bool last = j == P - 1 && kk[j] == nn[j] - 1;
-          const bool has_vor = !last && !pad[j] && (!kWave || tid + 1 < NT);
+          const bool has_vor = !last && !pad[j] && (!kWave || j + 1 < P || tid + 1 < NT);
           // the values of the next lanes
           auto load_next = [&](double (&xk1)[3], double (&xk2)[3], double (&vk1)[3], double (&qk1)[9], float (&dn)[3]) {
-            if constexpr (kWave) {
+            if constexpr (kWave && P == 1) {
 #pragma unroll
               for (int c = 0; c < 3; ++c) {
-                const double xn = lane_next(x[j][c]), vn = lane_next(v[j][c]);
-                xk1[c] = last ? xt[c] : xn;
+                const double vn = lane_next(v[j][c]);
+                xk1[c] = last ? xt[c] : xnext[c];
                 vk1[c] = last ? vt[c] : vn;
               }
 #pragma unroll
@@ -1071,6 +1085,20 @@ namespace erod {
                 geo[0][3] = len32(geo[0][0], geo[0][1], geo[0][2]);
                 geo[0][4] = lane_next(geo[0][3]);
               }
+              return;
+            }
+            if constexpr (kWave) {
+              // (the terms that use the next element's node difference have geo)
+              const bool next = j + 1 < P;
+              const int j1 = next ? j + 1 : 0;
+#pragma unroll
+              for (int c = 0; c < 3; ++c) {
+                const double vn = next ? v[j1][c] : lane_next(v[0][c]);
+                xk1[c] = last ? xt[c] : (next ? x[j1][c] : xnext[kWave ? c : 0]);
+                vk1[c] = last ? vt[c] : vn;
+              }
+#pragma unroll
+              for (int m = 0; m < 9; ++m) qk1[m] = next ? q[j1][m] : lane_next(q[0][m]);
               return;
             }
             if (last) {
@@ -1185,9 +1213,9 @@ namespace erod {
         if constexpr (kWave) {
 #pragma unroll
           for (int c = 0; c < 3; ++c) {
-            before[kWave ? c : 0] = lane_prev(mid[0].c[c]);
-            before[kWave ? 3 + c : 0] = lane_prev(mid[0].P[c]);
-            before[kWave ? 6 + c : 0] = lane_prev(mid[0].Rv[c]);
+            before[kWave ? c : 0] = lane_prev(mid[P - 1].c[c]);
+            before[kWave ? 3 + c : 0] = lane_prev(mid[P - 1].P[c]);
+            before[kWave ? 6 + c : 0] = lane_prev(mid[P - 1].Rv[c]);
           }
         } else {
 #pragma unroll
@@ -1210,7 +1238,7 @@ namespace erod {
           R cm[3], Pm[3], Rm[3];
 #pragma unroll
           for (int c = 0; c < 3; ++c) {
-            if constexpr (kWave) {
+            if (kWave && j == 0) {
               cm[c] = before[kWave ? c : 0];
               Pm[c] = before[kWave ? 3 + c : 0];
               Rm[c] = before[kWave ? 6 + c : 0];
@@ -1505,7 +1533,7 @@ namespace erod {
     struct Shape {
       int P, NT;
     };
-    constexpr Shape kShapes[] = {{1, 64}, {1, 128}, {1, 256}, {1, 512}, {2, 256}, {2, 512}, {4, 128}, {4, 256}};
+    constexpr Shape kShapes[] = {{1, 64}, {1, 128}, {1, 256}, {1, 512}, {2, 256}, {2, 512}, {4, 128}, {4, 256}, {2, 64}};
     constexpr int kNShapes = sizeof(kShapes) / sizeof(kShapes[0]);
 
     template <typename R>
@@ -1520,6 +1548,7 @@ namespace erod {
         case 5: return launch_tiles<R, 2, 512>(b, C, steps, g, in, out, t, st);
         case 6: return launch_tiles<R, 4, 128>(b, C, steps, g, in, out, t, st);
         case 7: return launch_tiles<R, 4, 256>(b, C, steps, g, in, out, t, st);
+        case 8: return launch_tiles<R, 2, 64>(b, C, steps, g, in, out, t, st);
         default: set_error("bad tile shape"); return EROD_ERR_INVALID;
       }
     }

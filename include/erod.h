@@ -178,7 +178,9 @@ int erod_set_rod_time(erod_batch* b, const double* time_per_rod);
  * an autotune, a batch takes the smallest capacity that holds its longest rod
  * (one element per thread up to 256 lanes, two from 1024; at 512 two for
  * FP32-bulk batches of more tiles than the device has compute units, one
- * otherwise); rods longer than the tile run as pieces
+ * otherwise; FP32-bulk batches that fill the device take two elements per
+ * thread in 128 lanes for rods of up to 128 elements, in 512 for rods of up to
+ * 256); rods longer than the tile run as pieces
  * (erod_set_fused_pieces).  Results do not depend on the shape. */
 int erod_set_fused_config(erod_batch* b, int lanes_per_tile, int elements_per_thread, int steps_per_launch);
 int erod_get_fused_config(const erod_batch* b, int* lanes_per_tile, int* elements_per_thread, int* steps_per_launch);
