@@ -325,14 +325,16 @@ namespace erod {
     }
     for (uint64_t i = 0; i < m; ++i) {
       const uint64_t a = i * n / m, z = (i + 1) * n / m;  // owned [a, z)
-      const uint64_t lo = i == 0 ? 0 : a - halo, hi = i + 1 == m ? n : z + halo;
+      // (a halo longer than the parts reaches past its neighbours', to the rod's
+      // end at most)
+      const uint64_t lo = a < halo ? 0 : a - halo, hi = std::min(n, z + halo);
       Seg sg{};
       sg.rod = rod;
       sg.off = uint32_t(lo);
       sg.n = uint32_t(hi - lo);
       sg.w0 = uint32_t(a - lo);
       sg.w1 = uint32_t(z - lo);
-      sg.ends = (i == 0 ? kSegFirst : 0u) | (i + 1 == m ? kSegLast : 0u);
+      sg.ends = (lo == 0 ? kSegFirst : 0u) | (hi == n ? kSegLast : 0u);
       out.push_back(sg);
     }
   }

@@ -763,8 +763,10 @@ namespace erod {
           if ((i < r_n[j] ? i : r_n[j] - 1) == g) rflags[j] |= uint32_t(k + 1) << 12;
         }
         own[j] = valid[j] && uint32_t(kk[j]) >= w0 && uint32_t(kk[j]) < w1;
-        clockw[j] = valid[j] && kk[j] == 0 && (!kSegs || (ends & kSegLast) != 0);
-        if (j == P - 1 && valid[j] && kk[j] == int(segn) - 1) tailw = (ends & kSegLast) != 0;
+        // (of the pieces that reach the rod's end, the one that owns its last element)
+        const bool ends_rod = (ends & kSegLast) != 0 && w1 == segn;
+        clockw[j] = valid[j] && kk[j] == 0 && ends_rod;
+        if (j == P - 1 && valid[j] && kk[j] == int(segn) - 1) tailw = ends_rod;
         // damping rates: one per rod, or (flag bit 2) per node and element
         const bool per_node = (r_fl[j] & 4u) != 0 && valid[j];
         gfj[j] = per_node ? C.gf[slot[j]] : static_cast<R>(r_gf[j]);
