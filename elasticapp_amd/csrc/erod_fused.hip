@@ -312,17 +312,22 @@ namespace erod {
     return order;
   }
 
+  // how many pieces `cut` makes of a rod of n elements: the least number of an
+  // even split whose longest piece, a middle part plus two halos, fits
+  static uint64_t n_pieces(uint64_t n, uint64_t cap, uint64_t halo) {
+    uint64_t m = 2;
+    while (true) {
+      const uint64_t part = (n + m - 1) / m;
+      if (part + 2 * halo <= cap || part <= 1) return m;
+      ++m;
+    }
+  }
+
   // The pieces of a rod of n elements for tiles of `cap` lanes: owned parts
   // of nearly equal length, each piece loading `halo` more elements on each
   // side that has a neighbouring piece; every piece at most cap long.
   static void cut(uint32_t rod, uint64_t n, uint64_t cap, uint64_t halo, std::vector<Seg>& out) {
-    uint64_t m = 2;
-    while (true) {
-      // the longest piece of an even split into m: a middle part plus two halos
-      const uint64_t part = (n + m - 1) / m;
-      if (part + 2 * halo <= cap || part <= 1) break;
-      ++m;
-    }
+    const uint64_t m = n_pieces(n, cap, halo);
     for (uint64_t i = 0; i < m; ++i) {
       const uint64_t a = i * n / m, z = (i + 1) * n / m;  // owned [a, z)
       // (a halo longer than the parts reaches past its neighbours', to the rod's
@@ -337,6 +342,28 @@ namespace erod {
       sg.ends = (lo == 0 ? kSegFirst : 0u) | (hi == n ? kSegLast : 0u);
       out.push_back(sg);
     }
+  }
+
+  // The halo of the pieces where the caller left their shape free: as wide as
+  // leaves every piece a CU of its own (beside the whole rods' tiles), up to
+  // 64, a launch taking as many steps.  Until then wider halos cost no time,
+  // and longer launches save it (a launch costs 20 us beside its steps): 24
+  // rods of 2,500 to 6,000 elements, us a step FP32-bulk 3.75 -> 2.31, FP64 7.7
+  // -> 4.95; 3 rods of 1,200 to 1,500 2.2 -> 1.64 and 3.6 -> 2.90.  FP32-bulk's runs stay `halo` / 2 steps, so results don't depend on it.
+  static uint64_t wide_halo(const erod_batch* b, int main_shape, uint64_t pcap, uint64_t halo) {
+    const uint64_t step = halo / 2, cap = uint64_t(fused_shape_lanes(main_shape));
+    uint64_t wide = halo, whole = 0;
+    for (uint64_t r = 0; r < b->n_rods; ++r)
+      if (planned(b, r) && !cut_rod(b, b->n_active[r], main_shape)) whole += b->n_active[r];
+    const uint64_t beside = (whole + cap - 1) / cap;
+    for (uint64_t h = halo; h <= 64 && 4 * h <= pcap; h += step) {
+      uint64_t pieces = beside;
+      for (uint64_t r = 0; r < b->n_rods && pieces <= uint64_t(b->cus); ++r)
+        if (planned(b, r) && cut_rod(b, b->n_active[r], main_shape)) pieces += n_pieces(b->n_active[r], pcap, h);
+      if (pieces > uint64_t(b->cus)) break;
+      wide = h;
+    }
+    return wide;
   }
 
   // Device copy of one group.  The arrays grow to the largest plan seen and
@@ -398,6 +425,7 @@ namespace erod {
     std::vector<uint32_t> len(b->n_rods), whole;
     std::vector<uint32_t> seg_rods;
     std::vector<Seg> segs;
+    const uint64_t wide = b->plan.seg_lanes == 0 && halo == 16 && shapes_free(b) ? wide_halo(b, si, pcap, halo) : halo;
     for (uint32_t i = 0; i < b->n_rods; ++i) {
       if (!planned(b, i)) continue;
       len[i] = static_cast<uint32_t>(b->n_active[i]);
@@ -407,7 +435,7 @@ namespace erod {
           return EROD_ERR_INVALID;
         }
         seg_rods.push_back(i);
-        cut(i, b->n_active[i], pcap, halo, segs);
+        cut(i, b->n_active[i], pcap, wide, segs);
       } else {
         whole.push_back(i);
       }
@@ -484,7 +512,7 @@ namespace erod {
     // became 7: 24 rods of 2,500 to 6,000 elements 6.05 -> 5.08 us a step
     // (FP32-bulk), 2,048 ragged rods 29.6 -> 28.0 (FP64, long rods in pieces)
     gs.run_steps = int(halo / 2);
-    gs.max_steps = 2 * gs.run_steps;
+    gs.max_steps = int(wide / (halo / 2)) * gs.run_steps;
     if (segs.empty()) gs.shape = -1;
     pl.precision = precision;
     pl.main_shape = si;
