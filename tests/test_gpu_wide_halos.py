@@ -24,14 +24,14 @@ def test_wide_halos(lengths, precision):
     assert halo == 16 and pieces >= 2
     ref.set_fused_pieces(lanes, epl, 16)  # (requested: the halo stays; no rod between 256 and 1,024, which it would cut)
     ref.step_fused(1, precision)
+    # (wider halos make more pieces; 25 rods leave no room for any)
+    assert pieces == ref.fused_pieces()[4] if len(lengths) == 25 else pieces > ref.fused_pieces()[4]
     for k, n in enumerate((15, 64, 133)):
         for b in (wide, ref):
             if k == 2:
                 b.set_step_budget(0, 77)
                 b.set_step_budget(len(lengths) - 1, 20)
             b.step_fused(n, precision)
-    if len(lengths) == 25:
-        assert pieces == ref.fused_pieces()[4]  # (no room for wider ones)
     for r in range(len(lengths)):
         for tag in STATE:
             assert np.array_equal(wide.get_rod(tag, r), ref.get_rod(tag, r)), (r, tag)
