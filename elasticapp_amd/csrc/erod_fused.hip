@@ -137,6 +137,18 @@ namespace erod {
   constexpr int kShape256 = 2, kShape512 = 3;      // one element per thread
   constexpr int kShape128x2 = 8, kShape512x2 = 4;  // two
 
+  // whether the second state copy that pieces need is there, or can be without
+  // taking the last of the memory
+  static bool shadow_fits(const erod_batch* b) {
+    if (b->d_shadow[3]) return true;
+    size_t free = 0, total = 0;
+    if (hipMemGetInfo(&free, &total) != hipSuccess) {
+      (void)hipGetLastError();
+      return false;
+    }
+    return free / 4 > 18 * sizeof(double) * b->E;
+  }
+
   // Default shape without measurement: the smallest capacity that holds the
   // longest rod; one element per thread up to 256 lanes, two elements per
   // thread for 1024 lanes; rods longer than 1024 elements run as pieces.  (Four
@@ -154,6 +166,15 @@ namespace erod {
   // step against 13.9; 1,024: 1.87 and 1.93; 512: 1.81 and 1.62; rods of 64:
   // 8,192 5.25 and 6.28, 3,072 2.84 and 3.01, 2,048 1.90 and 1.69), rods of up
   // to 256 in 512-lane ones (4,096 of 256: 11.2 and 13.3; 512: 2.41 and 2.02).
+  // Fused FP64 pays 8 waves' exchanges in 512-lane tiles: in a batch of few
+  // rods those past 256 elements run as pieces in 256 lanes (61 rods of up to
+  // 301: 4.6 -> 3.4 us a step; 100 of up to 512, over the line: 4.6 and 4.8).
+  // Not where launches are shorter than a halo, each of which passes over the
+  // state twice more (in launches of 8 steps 5.4 and 8.4).  Results are the
+  // same, bit by bit; FP32-bulk's depend on where a launch ends, so its rods
+  // stay whole.  (Batches with rods of 513 to 1,024 elements would gain more,
+  // 13.6 -> 3.5 for 20 of them, but take 1024 lanes by promise: an autotune, or
+  // a request for pieces, has them faster.)
   // A shape the autotuner chose is taken again while it stays feasible (a
   // replan after rods changed length keeps it, with its second group).
   static int default_shape(const erod_batch* b, int precision) {
@@ -165,6 +186,10 @@ namespace erod {
         maxn = std::max<uint64_t>(maxn, b->n_active[r]);
         lanes += b->n_active[r];
       }
+    const int launch = b->plan.steps_per_launch > 0 ? b->plan.steps_per_launch : 100;
+    if (precision == EROD_FP64 && shapes_free(b) && b->plan.seg_lanes == 0 && launch >= b->plan.halo &&
+        maxn > 256 && maxn <= 512 && lanes <= 32 * uint64_t(b->cus) && shadow_fits(b))
+      return kShape256;
     for (int si : pref)
       if (uint64_t(fused_shape_lanes(si)) >= maxn && shape_feasible(b, si)) {
         const bool two = fused_shape_lanes(si) == 512 && fused_shape_epl(si) == 2;
@@ -199,7 +224,9 @@ namespace erod {
       return -2;
     }
     const uint64_t halo = uint64_t(b->plan.halo);
-    if (!shapes_free(b) || fused_shape_lanes(main_shape) != 1024 || 2 * halo + 64 > 256) return main_shape;
+    if (!shapes_free(b) || 2 * halo + 64 > 256 ||
+        (fused_shape_lanes(main_shape) != 1024 && (precision != EROD_FP64 || main_shape != kShape256)))
+      return main_shape;
     uint64_t pieces256 = 0, pieces512 = 0;
     for (uint64_t r = 0; r < b->n_rods; ++r)
       if (planned(b, r) && cut_rod(b, b->n_active[r], main_shape)) {

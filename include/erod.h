@@ -180,7 +180,8 @@ int erod_set_rod_time(erod_batch* b, const double* time_per_rod);
  * FP32-bulk batches of more tiles than the device has compute units, one
  * otherwise; FP32-bulk batches that fill the device take two elements per
  * thread in 128 lanes for rods of up to 128 elements, in 512 for rods of up to
- * 256); rods longer than the tile run as pieces
+ * 256; small FP64 batches whose longest rod has 257 to 512 elements take 256
+ * lanes unless steps_per_launch is below 16); rods longer than the tile run as pieces
  * (erod_set_fused_pieces).  Results do not depend on the shape. */
 int erod_set_fused_config(erod_batch* b, int lanes_per_tile, int elements_per_thread, int steps_per_launch);
 int erod_get_fused_config(const erod_batch* b, int* lanes_per_tile, int* elements_per_thread, int* steps_per_launch);
@@ -202,7 +203,8 @@ int erod_get_fused_split(const erod_batch* b, int* lanes_per_tile, int* elements
  * from the state they had when the launch began, so that pieces need no
  * exchange within a launch; a launch over pieces then takes at most halo (or
  * halo - 1, if odd) steps, and the pieces' group is launched as often as
- * needed.  Results do not depend on the cut (bitwise).  For rods longer than any tile (the
+ * needed.  (Where neither shape nor halo was requested, halos widen to up to 64
+ * elements while every piece has a compute unit of its own.)  Results do not depend on the cut (bitwise).  For rods longer than any tile (the
  * reference's blocks emplace rods of any length, Block.hpp:568-611) and for
  * fused FP64, whose long-rod tiles spill registers.  The getter reports the
  * pieces' shape, halo, tiles and pieces in the current plan (0 if none). */

@@ -19,10 +19,11 @@ def _same(a, b):
 @pytest.mark.parametrize("precision", [FP64, FP32_BULK])
 @pytest.mark.parametrize("lengths,config,pieces", [
     ([256, 3], {FP64: (256, 1), FP32_BULK: (256, 1)}, {FP64: 0, FP32_BULK: 0}),
-    ([257, 3, 40], {FP64: (512, 1), FP32_BULK: (512, 1)}, {FP64: 0, FP32_BULK: 0}),
-    ([512, 2, 511], {FP64: (512, 1), FP32_BULK: (512, 1)}, {FP64: 0, FP32_BULK: 0}),
+    ([257, 3, 40], {FP64: (256, 1), FP32_BULK: (512, 1)}, {FP64: 256, FP32_BULK: 0}),
+    ([512, 2, 511], {FP64: (256, 1), FP32_BULK: (512, 1)}, {FP64: 256, FP32_BULK: 0}),
     ([400] * 400, {FP64: (512, 1), FP32_BULK: (512, 2)}, {FP64: 0, FP32_BULK: 0}),  # more than 256 tiles
     ([513, 20], {FP64: (1024, 2), FP32_BULK: (1024, 2)}, {FP64: 0, FP32_BULK: 0}),
+    ([400] * 21 + [20], {FP64: (512, 1), FP32_BULK: (512, 1)}, {FP64: 0, FP32_BULK: 0}),
     ([1025], {FP64: (0, 0), FP32_BULK: (0, 0)}, {FP64: 256, FP32_BULK: 256}),
     ([5000] * 20, {FP64: (0, 0), FP32_BULK: (0, 0)}, {FP64: 512, FP32_BULK: 512}),
     ([5000] * 32 + [700], {FP64: (1024, 2), FP32_BULK: (1024, 2)}, {FP64: 256, FP32_BULK: 1024}),
