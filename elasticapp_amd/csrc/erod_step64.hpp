@@ -132,15 +132,32 @@ namespace erod {
       rotate(q, rotation(w, c));
     }
 
+    // math::acos, for angles below 60 degrees with a root and a division that
+    // need no range test: z = (1 - x) / 2 is zero (then y is no number, and the
+    // result zero) or 2^-54 and more, the remainder z - h h a multiple of 2^-104.
+    // With the quotient below: 1,024 rods of 64 elements, 500 steps 1.667 -> 1.614
+    // ms, a pass with the state read back.
+    __device__ __forceinline__ double acos(double x) {
+      if (!(x > 0.5 && x <= 1.0)) return math::acos(x);
+      const double z = (1.0 - x) * 0.5;
+      const double y = root<true>(z);
+      const double t = math::asin_tail(y, z);
+      if (!(y > 0.0)) return 0.0;
+      const double h = math::bits_head26(y);
+      const double c = over<true>(z - h * h, divisor<true>(y + h));
+      return 2.0 * (h + (c + t));
+    }
+
     // curvature between neighbouring directors: InvRotateDivideOp<scalar>
     // (InvRotateDivide/Scalar.hpp:26-110)
     template <bool kPlain>
     __device__ __forceinline__ void curvature(const double qc[9], const double qn[9], const Divisor& D0, double kap[3]) {
       const double tr = qc[0] * qn[0] + qc[1] * qn[1] + qc[2] * qn[2] + qc[3] * qn[3] + qc[4] * qn[4] +
                         qc[5] * qn[5] + qc[6] * qn[6] + qc[7] * qn[7] + qc[8] * qn[8];
-      const double theta = math::acos(0.5 * tr - (0.5 + 1e-10));
-      // (theta / 2 sin(theta) is zero, NaN or between 1/2 and 2^50)
-      const double st = over<kPlain>(0.5 * theta / math::sin(theta + 1e-14), D0);
+      const double theta = acos(0.5 * tr - (0.5 + 1e-10));
+      // (theta is zero, NaN or 2^-27 to pi, the sine 2^-54 and more either way:
+      // their quotient is zero, NaN or 1/2 to 2^54)
+      const double st = over<kPlain>(over<true>(0.5 * theta, divisor<true>(math::sin(theta + 1e-14))), D0);
       kap[0] = st * (-qc[3] * qn[6] - qc[4] * qn[7] - qc[5] * qn[8] + qc[6] * qn[3] + qc[7] * qn[4] + qc[8] * qn[5]);
       kap[1] = st * (qc[0] * qn[6] + qc[1] * qn[7] + qc[2] * qn[8] - qc[6] * qn[0] - qc[7] * qn[1] - qc[8] * qn[2]);
       kap[2] = st * (-qc[0] * qn[3] - qc[1] * qn[4] - qc[2] * qn[5] + qc[3] * qn[0] + qc[4] * qn[1] + qc[5] * qn[2]);
