@@ -422,10 +422,11 @@ namespace erod {
         out.unst[c] = jw[c] * rate;
       }
       // Voronoi k.  A rod's last element has none.  FP32-bulk computes the
-      // terms anyway: its constants hold B = 0, kappa0 = 0 and D0 = 1, its
-      // neighbour inputs are finite values of the next lane and its log map
-      // clamps its argument, so the couple M = B (kappa - kappa0) and both
-      // terms below are exactly zero, with no branch (which every wave with a
+      // terms anyway, from the next lane's values, and selects kappa = 0 and
+      // eps = 1 (its constants hold B = 0, kappa0 = 0 and D0 = 1), so that the
+      // couple M = B (kappa - kappa0) and both terms below are exactly zero
+      // whatever the next lane, another rod's, and the rod's own state hold,
+      // infinities and NaN among them, with no branch (which every wave with a
       // rod end in it would take both sides of).  The FP64 path keeps the
       // reference's acos(tr / 2 - 1/2 - 1e-10), which is not defined for a
       // relative rotation of pi (a rod's last director against an idle lane's
@@ -449,8 +450,10 @@ namespace erod {
           eps = over<kPlain>(D, D0);
           step64::curvature<kPlain>(qk, qk1, D0, kap);
         } else {
-          eps = D * K.iD0;
+          eps = has_vor ? D * K.iD0 : 1.0f;
           curvature32(qk, qk1, K.iD0, kap, kWave && !has_vor);
+#pragma unroll
+          for (int c = 0; c < 3; ++c) kap[c] = has_vor ? kap[c] : 0.0f;
         }
         R M[3];
 #pragma unroll

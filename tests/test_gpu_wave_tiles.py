@@ -68,3 +68,33 @@ def test_free_shapes_of_batches_that_fill_the_device(n, per_cu, small, full, pre
             b.step_fused(3, precision)
         assert blk.fused_config()[:2] == (full if more and precision == FP32_BULK else small)
         assert all(np.array_equal(blk.get_field(t), ref.get_field(t)) for t in STATE)
+
+
+@pytest.mark.parametrize("precision", [FP64, FP32_BULK])
+@pytest.mark.parametrize("env", ["none", "tilted"])
+@pytest.mark.parametrize("lanes,epl", [(64, 1), (128, 1), (256, 1), (512, 1), (128, 2), (512, 2), (1024, 2), (512, 4), (1024, 4)])
+def test_a_rod_of_no_numbers_leaves_its_tile_alone(lanes, epl, env, precision):
+    """Rods in one tile beside ones that went non-finite, at their ends or
+    inside, in any part of their state, keep the bits they have without them."""
+    wl = random_workload(0, 0, 0, seed=900 + lanes + epl, lengths=[7, 5, 9, 4, 11, 6, 13, 4, 5])
+    if env == "tilted":
+        wl.gravity = (0.0, 0.0, -9.81)
+        wl.contact = (1e2, 1.0, 0.3, 1.0, 0.0, 0.01, (0.0, 0.6, 0.8))
+    ref, blk = build_block(wl), build_block(wl)
+    for b in (ref, blk):
+        b.set_fused_config(lanes, epl, 0)
+    lost = {0: ("Director", 0, np.nan), 2: ("Position", -1, np.inf), 4: ("Velocity", 0, np.nan),
+            6: ("AngularVelocity", -1, -np.inf), 7: ("Position", 0, np.nan)}
+    for r, (tag, i, value) in lost.items():
+        a = blk.get_rod(tag, r)
+        a[:, i] = value
+        blk.set_rod(tag, r, a)
+    for steps in (1, 1, 12):
+        for b in (ref, blk):
+            b.step_fused(steps, precision)
+        for r in range(len(wl.n_elems)):
+            if r not in lost:
+                for tag in STATE:
+                    assert np.array_equal(blk.get_rod(tag, r), ref.get_rod(tag, r)), (steps, r, tag)
+    assert blk.fused_config()[:2] == (lanes, epl)
+    assert [bool(f) for f in blk.check_finite()] == [r in lost for r in range(len(wl.n_elems))]
