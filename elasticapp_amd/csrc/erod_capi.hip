@@ -32,6 +32,7 @@ namespace erod {
       d.erase(std::unique(d.begin(), d.end()), d.end());
       if (d.size() * 4 <= b->n_rods) {
         if (b->rod_stage_capacity < d.size()) {
+          const OnDevice here(b->device);
           EROD_HIP(hipStreamSynchronize(b->stream));
           if (b->d_rod_stage) EROD_HIP(hipFree(b->d_rod_stage));
           if (b->d_rod_stage_idx) EROD_HIP(hipFree(b->d_rod_stage_idx));
@@ -588,6 +589,7 @@ int erod_get_rod_active_length(const erod_batch* b, uint64_t rod, uint64_t* n) {
 
 static int ensure_budget_buffer(erod_batch* b) {
   if (b->d_steps_left) return EROD_OK;
+  const OnDevice here(b->device);
   EROD_HIP(hipMalloc(&b->d_steps_left, sizeof(uint32_t) * b->n_rods));
   b->budgets_dirty = true;
   return EROD_OK;

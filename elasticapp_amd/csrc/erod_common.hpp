@@ -248,6 +248,26 @@ namespace erod {
     if (_rc != EROD_OK) return _rc;                      \
   } while (0)
 
+  // Makes a batch's device current where memory or an event is made on first
+  // use, which may be on a thread, or after a call, that made another device
+  // current (launches and copies go by their stream); the caller's device is
+  // current again when this goes.
+  class OnDevice {
+  public:
+    explicit OnDevice(int device) {
+      moved_ = hipGetDevice(&was_) == hipSuccess && was_ != device && hipSetDevice(device) == hipSuccess;
+    }
+    ~OnDevice() {
+      if (moved_) (void)hipSetDevice(was_);
+    }
+    OnDevice(const OnDevice&) = delete;
+    OnDevice& operator=(const OnDevice&) = delete;
+
+  private:
+    int was_ = 0;
+    bool moved_ = false;
+  };
+
   constexpr int kThreads = 256;
   inline unsigned grid_for(uint64_t n) {
     uint64_t g = (n + kThreads - 1) / kThreads;

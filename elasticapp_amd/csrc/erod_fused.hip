@@ -550,6 +550,7 @@ namespace erod {
   }
 
   int fused_prepare(erod_batch* b, int precision) {
+    const OnDevice here(b->device);
     int rc = sync_rods(b);
     if (rc) return rc;
     FusedPlan& pl = b->plan;
@@ -639,6 +640,7 @@ namespace erod {
   // Unless the caller set a second group, each smaller shape is then tried as
   // one for the rods that find no room beside longer ones, and kept if faster.
   int fused_autotune(erod_batch* b, int precision, int trial_steps, double* best_ms) {
+    const OnDevice here(b->device);
     int rc = fused_prepare(b, precision);
     if (rc) return rc;
     const int snap_fields[4] = {EROD_POSITION, EROD_VELOCITY, EROD_DIRECTOR, EROD_ANGULAR_VELOCITY};

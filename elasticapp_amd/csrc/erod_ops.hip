@@ -818,6 +818,7 @@ namespace erod {
   // the second copy of the state and the slots' rods, for k_steps; false when
   // the device has no room for them
   static bool steps_buffers(erod_batch* b) {
+    const OnDevice here(b->device);
     static const int fields[4] = {EROD_POSITION, EROD_VELOCITY, EROD_DIRECTOR, EROD_ANGULAR_VELOCITY};
     bool ok = true;
     if (b->E + 1 > kThreads)

@@ -71,6 +71,7 @@ namespace erod {
   int serve_copy_rods(erod_batch* dst, const erod_batch* src, const std::vector<CopyPair>& pairs) {
     if (pairs.empty()) return EROD_OK;
     if (dst->copy_capacity < pairs.size()) {
+      const OnDevice here(dst->device);
       EROD_HIP(hipStreamSynchronize(dst->stream));
       if (dst->d_copy_pairs) EROD_HIP(hipFree(dst->d_copy_pairs));
       dst->d_copy_pairs = nullptr;

@@ -48,8 +48,10 @@ namespace erod {
     }
 
     // pinned memory of the batch, allocated on first use; null if there is none
-    void* pinned(void*& p, size_t bytes) {
-      if (!p && hipHostMalloc(&p, bytes, hipHostMallocDefault) != hipSuccess) {
+    void* pinned(const erod_batch* b, void*& p, size_t bytes) {
+      if (p) return p;
+      const OnDevice here(b->device);
+      if (hipHostMalloc(&p, bytes, hipHostMallocDefault) != hipSuccess) {
         p = nullptr;
         (void)hipGetLastError();
       }
@@ -57,6 +59,8 @@ namespace erod {
     }
 
     int ring_events(erod_batch* b) {
+      if (b->ring_ev[kRing - 1]) return EROD_OK;
+      const OnDevice here(b->device);
       for (int i = 0; i < kRing; ++i)
         if (!b->ring_ev[i]) EROD_HIP(hipEventCreateWithFlags(&b->ring_ev[i], hipEventDisableTiming));
       return EROD_OK;
@@ -191,7 +195,7 @@ namespace erod {
     const double* src = b->d_field[field] + slot;
     const size_t line = cnt * sizeof(double), bytes = line * nc;
     const bool whole = cnt == slots || nc == 1;
-    void* stage = bytes <= kStageBytes ? pinned(b->stage, kStageBytes) : pinned(b->ring, kRing * kChunk);
+    void* stage = bytes <= kStageBytes ? pinned(b, b->stage, kStageBytes) : pinned(b, b->ring, kRing * kChunk);
     if (stage && bytes < kRingFrom) {
       if (whole) {
         EROD_HIP(hipMemcpyAsync(stage, src, bytes, hipMemcpyDeviceToHost, b->stream));

@@ -1,0 +1,84 @@
+"""What the library does on the host, checked with no GPU: liberod.so runs over
+a stand-in for the HIP runtime (hip_double.cpp) that keeps memory on the host
+and logs allocations, copies and launches.  Each test is a short program in a
+process of its own."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+LIB = os.path.join(ROOT, "elasticapp_amd", "liberod.so")
+
+PRELUDE = """
+import ctypes, re, sys
+import numpy as np
+import elasticapp_amd as ea
+from elasticapp_amd import FP32_BULK, FP64, DeviceBlock
+D = ctypes.CDLL(sys.argv[1])
+D.double_log.restype = ctypes.c_char_p
+D.double_live.restype = ctypes.c_size_t
+
+def log(word=""):
+    return [l for l in D.double_log().decode().splitlines() if word in l]
+
+def launches():
+    # (precision, elements per thread, threads, pieces, tiles, steps) of every fused launch
+    return [(a[0], int(a[1]), int(a[2]), int(a[3]), int(a[4]), int(a[5])) for a in
+            re.findall(r"k_fusedI([df])Li(\\d+)ELi(\\d+)ELi\\d+ELb([01])E\\S* grid (\\d+) steps (\\d+)", D.double_log().decode())]
+
+def block(lengths):
+    b = DeviceBlock(list(lengths))
+    b.set_rod_dt(1e-5)
+    D.double_clear()
+    return b
+"""
+
+
+@pytest.fixture(scope="session")
+def run(tmp_path_factory):
+    if not os.path.exists(LIB):
+        if not os.path.exists("/opt/rocm/bin/hipcc"):
+            pytest.skip("liberod.so not built and no hipcc here")
+        from elasticapp_amd import build
+        build.build()
+    so = str(tmp_path_factory.mktemp("hip") / "hip_double.so")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-shared", "-fPIC", "-o", so,
+                    os.path.join(ROOT, "tests", "hip_double.cpp")], check=True)
+
+    def go(program):
+        env = dict(os.environ)
+        env["LD_PRELOAD"] = " ".join([so] + env.get("LD_PRELOAD", "").split())
+        r = subprocess.run([sys.executable, "-c", PRELUDE + program, so], cwd=ROOT, env=env, capture_output=True, text=True,
+                           timeout=120)
+        assert r.returncode == 0, r.stdout + r.stderr
+        return r.stdout
+
+    return go
+
+
+def test_memory_made_on_first_use_is_on_the_batchs_device(run):
+    """A program may make another device current between two calls on a batch:
+    what the calls allocate, and the events they record, are the batch's
+    device's, and the program's device is current again afterwards."""
+    run("""
+blk = block([400, 30])            # on device 0
+D.double_set_device(1)
+blk.step(1e-5, 30)                # second copy of the state
+blk.get_field("Position")         # pinned stage
+blk.step_fused(20, FP64)          # pieces: second copy, plan
+assert log("k_steps") and len(launches()) > 1
+assert all(l.endswith("foreign 0") for l in log("foreign")), log("foreign")
+big = block([70000])              # on device 1
+D.double_set_device(0)
+big.get_field("Director")         # ring and events
+big.autotune(FP32_BULK, 4)
+assert len(launches()) > 1
+assert all(l.endswith("foreign 0") for l in log("foreign")), log("foreign")
+d = ctypes.c_int()
+assert D.hipGetDevice(ctypes.byref(d)) == 0 and d.value == 0
+assert D.double_live(0) > 0 and D.double_live(1) > 0
+blk.close(); big.close()
+assert D.double_live(0) == 0 and D.double_live(1) == 0
+""")
