@@ -28,7 +28,9 @@ namespace erod {
     // operands met so far: bad if a divisor or radicand lies outside 2^-100 ...
     // 2^100, a numerator other than zero below 2^-800, or one above 2^600
     struct Range {
-      uint32_t least = 0xffffffffu;  // smallest (high word << 1) - 1; a zero's is the largest
+      // smallest exponent e, 2^(e-1) <= |n| < 2^e, denormal numbers' true one
+      // among them; a zero's, an infinity's and a NaN's is 0
+      int least = 0;
       bool out = false;
 
       __device__ __forceinline__ static uint32_t high(double v) { return static_cast<uint32_t>(__double2hiint(v)); }
@@ -36,10 +38,10 @@ namespace erod {
         out |= high(d) - ((1023u - 100u) << 20) >= (200u << 20);  // (a negative one, an infinity or a NaN too)
       }
       // a numerator known not to be large
-      __device__ __forceinline__ void numerator(double n) { least = min(least, (high(n) << 1) - 1u); }
+      __device__ __forceinline__ void numerator(double n) { least = min(least, __builtin_amdgcn_frexp_exp(n)); }
       // the largest magnitude of numerators that may be
       __device__ __forceinline__ void largest(double a) { out |= !(a < 0x1p600); }
-      __device__ __forceinline__ bool bad() const { return out || least < ((1023u - 800u) << 21); }
+      __device__ __forceinline__ bool bad() const { return out || least < -799; }
     };
 
     // a divisor with its reciprocal

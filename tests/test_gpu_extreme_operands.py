@@ -71,3 +71,31 @@ def test_both_forms_round_like_the_oracle(kind):
                 assert np.array_equal(plain.get_rod(tag, r), c, equal_nan=True), (n, r, tag)
     if kind in ("overflow", "nonfinite"):
         assert fused.check_finite()[[0, 2, 3]].all() and not fused.check_finite()[[1, 4, 5]].any()
+
+
+@pytest.mark.parametrize("scale", [1e-320, 1e-316, 1e-312, 1e-306])
+def test_denormal_numerators_between_ordinary_ones(scale):
+    """A stretched straight rod that spins by denormal rates: in its divisions
+    by the dilatation every numerator is zero, ordinary, or below 2^-1042, where
+    a plain division loses the last unit."""
+    from elasticapp_amd import straight_rod_state
+
+    rng = np.random.default_rng(5)
+    wl = random_workload(0, 0, 0, seed=602, forces=False, lengths=[60, 100])
+    for r, n in enumerate(wl.n_elems):
+        st = straight_rod_state(n, 0.02, 1.0, [0.0, 0.0, 0.0], [1.0, 0.0, 0.0], [0.0, 0.0, 1.0], 1000.0, 1e6, 4e5, 0.1, 0.1)
+        st["Position"] = st["Position"] * 1.3
+        st["Velocity"][0] = rng.normal(size=n + 1)
+        st["AngularVelocity"] = scale * rng.normal(size=(3, n))
+        wl.states[r] = st
+    sysm = oracle_system(wl, variant="devmath")
+    fused, plain = device_block(wl), device_block(wl)
+    for n in (1, 2, 10):
+        sysm.step(wl.dt, n)
+        fused.step_fused(n, FP64)
+        plain.step(wl.dt, n)
+        for r in range(len(wl.n_elems)):
+            for tag in STATE:
+                c = sysm.rod_field(r, tag)
+                assert np.array_equal(fused.get_rod(tag, r), c), (n, r, tag)
+                assert np.array_equal(plain.get_rod(tag, r), c), (n, r, tag)
