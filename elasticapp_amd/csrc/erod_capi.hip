@@ -604,6 +604,8 @@ int erod_set_rod_step_budget(erod_batch* b, uint64_t rod, uint64_t steps) {
     b->graph_precision = -1;
   }
   b->steps_left[rod] = v;
+  // (a graph captured so far reads no budgets)
+  if (!b->budgets) b->graph_precision = -1;
   b->budgets = true;
   b->budgets_dirty = true;
   return EROD_OK;

@@ -60,3 +60,24 @@ def test_alternating_precisions(lengths):
         assert _same(a, b), k
         assert np.array_equal(a.rod_time(), b.rod_time()), k
         assert a.fused_config() == b.fused_config() and a.fused_pieces() == b.fused_pieces(), k
+
+
+@pytest.mark.parametrize("precision", [FP64, FP32_BULK])
+@pytest.mark.parametrize("lengths", [[30, 200], [1300, 40]])
+def test_a_first_budget_after_a_capture(lengths, precision):
+    """A graph captured before any rod had a step budget is captured again once
+    one has."""
+    wl = random_workload(0, 0, 0, seed=40 + lengths[0], lengths=lengths)
+    a, b = build_block(wl), build_block(wl)
+    for blk in (a, b):
+        blk.set_fused_config(0, 0, 20)
+    a.capture_fused_graph(60, precision)
+    for n in (60, 120):
+        for blk in (a, b):
+            if n == 120:
+                blk.set_step_budget(0, 50)
+        a.step_fused_graph(n, 60, precision)
+        b.step_fused(n, precision)
+        assert _same(a, b), n
+        assert np.array_equal(a.rod_time(), b.rod_time()), n
+    assert a.rod_time()[0] < a.rod_time()[1]
