@@ -149,6 +149,9 @@ namespace erod {
     return free / 4 > 18 * sizeof(double) * b->E;
   }
 
+  // whether pieces of 256 lanes leave a part of 64 elements between their halos
+  static bool halo_fits_256(const erod_batch* b) { return 2 * b->plan.halo + 64 <= 256; }
+
   // Default shape without measurement: the smallest capacity that holds the
   // longest rod; one element per thread up to 256 lanes, two elements per
   // thread for 1024 lanes; rods longer than 1024 elements run as pieces.  (Four
@@ -187,7 +190,7 @@ namespace erod {
         lanes += b->n_active[r];
       }
     const int launch = b->plan.steps_per_launch > 0 ? b->plan.steps_per_launch : 100;
-    if (precision == EROD_FP64 && shapes_free(b) && b->plan.seg_lanes == 0 && launch >= b->plan.halo &&
+    if (precision == EROD_FP64 && shapes_free(b) && b->plan.seg_lanes == 0 && launch >= b->plan.halo && halo_fits_256(b) &&
         maxn > 256 && maxn <= 512 && lanes <= 32 * uint64_t(b->cus) && shadow_fits(b))
       return kShape256;
     for (int si : pref)
@@ -224,7 +227,7 @@ namespace erod {
       return -2;
     }
     const uint64_t halo = uint64_t(b->plan.halo);
-    if (!shapes_free(b) || 2 * halo + 64 > 256 ||
+    if (!shapes_free(b) || !halo_fits_256(b) ||
         (fused_shape_lanes(main_shape) != 1024 && (precision != EROD_FP64 || main_shape != kShape256)))
       return main_shape;
     uint64_t pieces256 = 0, pieces512 = 0;

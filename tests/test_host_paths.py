@@ -82,3 +82,17 @@ assert D.double_live(0) > 0 and D.double_live(1) > 0
 blk.close(); big.close()
 assert D.double_live(0) == 0 and D.double_live(1) == 0
 """)
+
+
+@pytest.mark.parametrize("halo,pieces", [(0, 1), (96, 1), (97, 0), (100, 0), (127, 0), (128, 0), (200, 0)])
+def test_small_fp64_batches_with_a_long_halo(run, halo, pieces):
+    """FP64 rods of 257 to 512 elements take pieces of 256 lanes only with a halo
+    that leaves them room; with a longer one they run whole, in 512."""
+    run("""
+blk = block([300, 400, 20])
+blk.set_fused_pieces(0, 0, %d)
+blk.set_fused_config(0, 0, 200)
+blk.step_fused(200, FP64)
+assert all(l[:3] == (("d", 1, 256) if %d else ("d", 1, 512)) for l in launches()), launches()
+assert any(l[3] for l in launches()) == %d
+""" % (halo, pieces, pieces))
