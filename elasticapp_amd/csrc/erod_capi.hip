@@ -528,7 +528,12 @@ int erod_set_rod_time(erod_batch* b, const double* t) {
   return EROD_OK;
 }
 
-static int fused_common(erod_batch* b, int precision) {
+static uint64_t steps_per_launch(const erod_batch* b) {
+  return b->plan.steps_per_launch > 0 ? uint64_t(b->plan.steps_per_launch) : 100;
+}
+
+// before a fused call whose longest run of steps without a break is `run`
+static int fused_common(erod_batch* b, int precision, uint64_t run) {
   if (precision != EROD_FP64 && precision != EROD_FP32_BULK) {
     set_error("unknown precision");
     return EROD_ERR_INVALID;
@@ -548,7 +553,7 @@ static int fused_common(erod_batch* b, int precision) {
     EROD_HIP(hipStreamSynchronize(b->stream));
     b->budgets_dirty = false;
   }
-  return fused_prepare(b, precision);
+  return fused_prepare(b, precision, std::min(run, steps_per_launch(b)));
 }
 
 // The kernel spends min(budget, s) steps of each planned rod's budget per
@@ -729,13 +734,13 @@ int erod_get_fused_config(const erod_batch* b, int* lanes, int* elements_per_thr
   const int si = b->plan.valid ? b->plan.g[0].shape : -1;
   if (lanes) *lanes = si >= 0 ? fused_shape_lanes(si) : 0;
   if (elements_per_thread) *elements_per_thread = si >= 0 ? fused_shape_epl(si) : 0;
-  if (steps) *steps = b->plan.steps_per_launch > 0 ? b->plan.steps_per_launch : 100;
+  if (steps) *steps = static_cast<int>(steps_per_launch(b));
   return EROD_OK;
 }
 
 int erod_autotune_fused(erod_batch* b, int precision, int trial_steps, double* best_ms_per_step) {
   if (check_batch(b) || trial_steps <= 0) return EROD_ERR_INVALID;
-  int rc = fused_common(b, precision);
+  int rc = fused_common(b, precision, uint64_t(trial_steps));
   if (rc) return rc;
   return fused_autotune(b, precision, trial_steps, best_ms_per_step);
 }
@@ -752,9 +757,9 @@ static int after_launch(erod_batch* b, uint64_t s) {
 
 int erod_step_fused(erod_batch* b, int precision, uint64_t n) {
   if (check_batch(b)) return EROD_ERR_INVALID;
-  int rc = fused_common(b, precision);
+  int rc = fused_common(b, precision, n);
   if (rc) return rc;
-  const uint64_t spl = b->plan.steps_per_launch > 0 ? uint64_t(b->plan.steps_per_launch) : 100;
+  const uint64_t spl = steps_per_launch(b);
   uint64_t done = 0;
   b->last_launches = 0;
   EROD_HIP(hipEventRecord(b->ev0, b->stream));
@@ -775,7 +780,7 @@ int erod_step_fused(erod_batch* b, int precision, uint64_t n) {
 // (a chunk that is a multiple of the interval starts every replay at the
 // same phase; otherwise a replay at another phase captures again)
 static int ensure_graph(erod_batch* b, int precision, uint64_t chunk) {
-  const uint64_t spl = b->plan.steps_per_launch > 0 ? uint64_t(b->plan.steps_per_launch) : 100;
+  const uint64_t spl = steps_per_launch(b);
   const bool same_schedule =
       b->graph_reortho[0] == b->reortho_every && (b->reortho_every == 0 || b->graph_reortho[1] == b->reortho_phase);
   if (b->graph_precision != precision || b->graph_chunk != chunk || !b->graph_exec || !same_schedule) {
@@ -829,7 +834,7 @@ int erod_capture_fused_graph(erod_batch* b, int precision, uint64_t chunk) {
     set_error("erod_capture_fused_graph: chunk must be positive");
     return EROD_ERR_INVALID;
   }
-  int rc = fused_common(b, precision);
+  int rc = fused_common(b, precision, chunk);
   return rc ? rc : ensure_graph(b, precision, chunk);
 }
 
@@ -838,9 +843,9 @@ int erod_step_fused_graph(erod_batch* b, int precision, uint64_t n, uint64_t chu
     set_error("erod_step_fused_graph: chunk must be positive");
     return EROD_ERR_INVALID;
   }
-  int rc = fused_common(b, precision);
+  int rc = fused_common(b, precision, std::min(n, chunk));
   if (rc) return rc;
-  const uint64_t spl = b->plan.steps_per_launch > 0 ? uint64_t(b->plan.steps_per_launch) : 100;
+  const uint64_t spl = steps_per_launch(b);
   const uint64_t whole = n / chunk, rest = n % chunk;
   if (whole > 0 && (rc = ensure_graph(b, precision, chunk))) return rc;
   EROD_HIP(hipEventRecord(b->ev0, b->stream));

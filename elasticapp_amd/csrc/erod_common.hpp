@@ -142,10 +142,12 @@ namespace erod {
     // groups: 0 main, 1 second (short rods), 2 pieces of long rods
     TileGroup g[3];
     bool valid = false;
-    // where the caller leaves the shapes free they depend on the precision:
-    // the precision, main shape and pieces' shape of g, and the plan of the
-    // other precision, kept while both are in use
+    // where the caller leaves the shapes free they depend on the precision and
+    // on whether the call's launches are shorter than a halo: both, the main
+    // shape and pieces' shape of g, and the plan of the other calls, kept while
+    // both are in use
     int precision = -1, main_shape = -1, piece_shape = -1;
+    bool brief = false;
     struct Kept {
       TileGroup g[3];
       bool valid = false;
@@ -291,7 +293,8 @@ namespace erod {
   int ops_apply_pre_dynamic(erod_batch* b, double time);
   int ops_apply_post_dynamic(erod_batch* b);
   // fused path (erod_fused.hip)
-  int fused_prepare(erod_batch* b, int precision);
+  // launch: steps of the longest launch to come
+  int fused_prepare(erod_batch* b, int precision, uint64_t launch);
   int fused_launch(erod_batch* b, int precision, int steps, bool timed);
   int fused_reorthonormalize(erod_batch* b);
   // the directors of every rod with steps left to take (no budget, or one

@@ -172,15 +172,16 @@ namespace erod {
   // Fused FP64 pays 8 waves' exchanges in 512-lane tiles: in a batch of few
   // rods those past 256 elements run as pieces in 256 lanes (61 rods of up to
   // 301: 4.6 -> 3.4 us a step; 100 of up to 512, over the line: 4.6 and 4.8).
-  // Not where launches are shorter than a halo, each of which passes over the
-  // state twice more (in launches of 8 steps 5.4 and 8.4).  Results are the
+  // Not for calls whose launches are shorter than a halo, each of which passes
+  // over the state twice more (calls on one rod of 300, us: 1 step 16 whole and
+  // 25 in pieces, 8 steps 44 and 44, 16 steps 75 and 63, 100 steps 402 and 274).  Results are the
   // same, bit by bit; FP32-bulk's depend on where a launch ends, so its rods
   // stay whole.  (Batches with rods of 513 to 1,024 elements would gain more,
   // 13.6 -> 3.5 for 20 of them, but take 1024 lanes by promise: an autotune, or
   // a request for pieces, has them faster.)
   // A shape the autotuner chose is taken again while it stays feasible (a
   // replan after rods changed length keeps it, with its second group).
-  static int default_shape(const erod_batch* b, int precision) {
+  static int default_shape(const erod_batch* b, int precision, bool brief) {
     static const int pref[] = {0, 1, 2, 4, 5, 3, 7, 6, 8};
     if (b->plan.tuned_shape >= 0 && shape_feasible(b, b->plan.tuned_shape)) return b->plan.tuned_shape;
     uint64_t maxn = 0, lanes = 0;
@@ -189,9 +190,8 @@ namespace erod {
         maxn = std::max<uint64_t>(maxn, b->n_active[r]);
         lanes += b->n_active[r];
       }
-    const int launch = b->plan.steps_per_launch > 0 ? b->plan.steps_per_launch : 100;
-    if (precision == EROD_FP64 && shapes_free(b) && b->plan.seg_lanes == 0 && launch >= b->plan.halo && halo_fits_256(b) &&
-        maxn > 256 && maxn <= 512 && lanes <= 32 * uint64_t(b->cus) && shadow_fits(b))
+    if (precision == EROD_FP64 && shapes_free(b) && b->plan.seg_lanes == 0 && !brief && halo_fits_256(b) && maxn > 256 &&
+        maxn <= 512 && lanes <= 32 * uint64_t(b->cus) && shadow_fits(b))
       return kShape256;
     for (int si : pref)
       if (uint64_t(fused_shape_lanes(si)) >= maxn && shape_feasible(b, si)) {
@@ -552,14 +552,15 @@ namespace erod {
     return EROD_OK;
   }
 
-  int fused_prepare(erod_batch* b, int precision) {
+  int fused_prepare(erod_batch* b, int precision, uint64_t launch) {
     const OnDevice here(b->device);
     int rc = sync_rods(b);
     if (rc) return rc;
     FusedPlan& pl = b->plan;
     if (!pl.valid) pl.kept.valid = false;  // the rods changed: so did its
-    if (!pl.valid || pl.precision != precision) {
-      const int si = default_shape(b, precision);
+    const bool brief = launch < uint64_t(pl.halo);
+    if (!pl.valid || pl.precision != precision || pl.brief != brief) {
+      const int si = default_shape(b, precision, brief);
       if (si < 0) {
         set_error("no fused tile shape holds this batch (a requested shape with more elements per thread than "
                   "a rod has)");
@@ -567,7 +568,7 @@ namespace erod {
       }
       const int ps = piece_shape(b, si, precision);
       if (pl.valid && (si != pl.main_shape || ps != pl.piece_shape)) {
-        // the other precision's shapes: its plan comes in, this one is kept
+        // other shapes than this plan's: the kept one comes in, this one is kept
         for (int k = 0; k < 3; ++k) std::swap(pl.g[k], pl.kept.g[k]);
         std::swap(pl.main_shape, pl.kept.main_shape);
         std::swap(pl.piece_shape, pl.kept.piece_shape);
@@ -576,6 +577,7 @@ namespace erod {
       }
       if (!pl.valid && (rc = plan_tiles(b, si, ps, precision))) return rc;
       pl.precision = precision;
+      pl.brief = brief;
     }
     if (precision == EROD_FP32_BULK && b->const32_dirty) {
       const uint64_t total = const32_offset(b, kNConst32);
@@ -644,7 +646,7 @@ namespace erod {
   // one for the rods that find no room beside longer ones, and kept if faster.
   int fused_autotune(erod_batch* b, int precision, int trial_steps, double* best_ms) {
     const OnDevice here(b->device);
-    int rc = fused_prepare(b, precision);
+    int rc = fused_prepare(b, precision, uint64_t(trial_steps));
     if (rc) return rc;
     const int snap_fields[4] = {EROD_POSITION, EROD_VELOCITY, EROD_DIRECTOR, EROD_ANGULAR_VELOCITY};
     // snapshot buffers and the plan settings the trials change, released and

@@ -96,3 +96,28 @@ blk.step_fused(200, FP64)
 assert all(l[:3] == (("d", 1, 256) if %d else ("d", 1, 512)) for l in launches()), launches()
 assert any(l[3] for l in launches()) == %d
 """ % (halo, pieces, pieces))
+
+
+def test_short_fp64_calls_keep_small_batches_whole(run):
+    """Pieces cost a launch two passes over the state more: a call whose launches
+    are shorter than a halo runs rods of 257 to 512 elements whole, also between
+    longer calls, and each kind's plan is made once."""
+    run("""
+blk = block([300, 400, 270])
+def pieces(n, graph=0):
+    D.double_clear()
+    blk.step_fused_graph(n, graph, FP64) if graph else blk.step_fused(n, FP64)
+    ls = launches()
+    assert ls and len({l[3] for l in ls}) == 1
+    return ls[0][3]
+assert [pieces(n) for n in (1, 8, 15)] == [0, 0, 0]
+assert len(launches()) == 1 and not log("k_copy_cut_state")
+assert [pieces(n) for n in (16, 100, 5, 200)] == [1, 1, 0, 1]
+for n, p in ((8, 0), (64, 1), (8, 0)):
+    assert pieces(n) == p and not log("copy device")  # (no plan goes up again)
+assert pieces(90, 8) == 0 and pieces(90, 30) == 1 and pieces(8, 30) == 0
+blk.step_fused_graph(90, 30, FP64)
+assert len(log("replay")) == 3 and not log("capture")  # (the graph of 30 steps is still that plan's)
+blk.set_fused_config(0, 0, 8)
+assert pieces(100) == 0
+""")
