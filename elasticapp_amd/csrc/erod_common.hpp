@@ -160,6 +160,7 @@ namespace erod {
 struct erod_batch {
   int device = 0;
   int cus = 256;  // compute units of the device
+  bool pool = false;  // a server's pool, whose memory its HBM budget bounds
   hipStream_t stream = nullptr;
   uint64_t n_rods = 0;
   uint64_t E = 0;  // element slots incl. ghosts

@@ -211,6 +211,7 @@ namespace {
       erod_batch_destroy(p);
       return rc;
     }
+    p->pool = true;
     for (uint64_t r = 0; r < p->n_rods; ++r) empty_slot(p, r);
     p->all_full = false;
     p->damping_dirty = false;  // empty slots carry no damping; copied rods bring their rates

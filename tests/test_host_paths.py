@@ -121,3 +121,22 @@ assert len(log("replay")) == 3 and not log("capture")  # (the graph of 30 steps 
 blk.set_fused_config(0, 0, 8)
 assert pieces(100) == 0
 """)
+
+
+@pytest.mark.parametrize("precision", ["FP64", "FP32_BULK"])
+def test_a_pool_stays_within_its_hbm_budget(run, precision):
+    """What a server allocates for rods of 257 to 512 elements, from its first
+    request to the last, is what it reports."""
+    run("""
+lib = block([300, 400, 270, 500])
+before = D.double_live(0)
+srv = ea.Server(lib, [(512, 400)], %s, 20)
+for i in range(6):
+    srv.submit(i, [0, 1, 2, 3][: 1 + i %% 4], 40)
+done = []
+while len(done) < 6:
+    done += srv.tick()
+used, said = D.double_live(0) - before, srv.status()["pool_bytes"]
+assert used <= 1.02 * said, (used, said)  # (tables of a few KB beside the fields)
+assert launches() and not any(l[3] for l in launches())
+""" % precision)
