@@ -560,7 +560,8 @@ namespace erod {
     if (rc) return rc;
     FusedPlan& pl = b->plan;
     if (!pl.valid) pl.kept.valid = false;  // the rods changed: so did its
-    const bool brief = launch < uint64_t(pl.halo);
+    // (the calls' lengths decide on free shapes only)
+    const bool brief = precision == EROD_FP64 && shapes_free(b) && launch < uint64_t(pl.halo);
     if (!pl.valid || pl.precision != precision || pl.brief != brief) {
       const int si = default_shape(b, precision, brief);
       if (si < 0) {

@@ -140,3 +140,20 @@ used, said = D.double_live(0) - before, srv.status()["pool_bytes"]
 assert used <= 1.02 * said, (used, said)  # (tables of a few KB beside the fields)
 assert launches() and not any(l[3] for l in launches())
 """ % precision)
+
+
+def test_a_tuned_plan_outlives_calls_of_another_length(run):
+    """The plan an autotune leaves in place stands for calls longer and shorter
+    than its trials, also where the caller had requested another shape."""
+    run("""
+for precision, fast in ((FP32_BULK, b"k_fusedIfLi1ELi256E"), (FP64, b"k_fusedIdLi1ELi256E")):
+    for lanes in (0, 512):
+        blk = block([200, 250, 30, 100])
+        blk.set_fused_config(lanes, 0, 0)
+        D.double_fast(fast)
+        blk.autotune(precision, 4)
+        for n in (100, 3, 100):
+            D.double_clear()
+            blk.step_fused(n, precision)
+            assert [l[1:3] for l in launches()] == [(1, 256)], (precision, lanes, n, launches())
+""")
