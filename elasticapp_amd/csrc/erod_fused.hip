@@ -129,10 +129,11 @@ namespace erod {
     return true;
   }
 
-  // whether neither the caller nor the autotuner chose the main shape
-  static bool shapes_free(const erod_batch* b) {
-    return b->plan.lanes_per_tile == 0 && b->plan.elements_per_thread == 0 && b->plan.tuned_shape < 0;
-  }
+  // whether the caller left the main shape free
+  static bool unrequested(const erod_batch* b) { return b->plan.lanes_per_tile == 0 && b->plan.elements_per_thread == 0; }
+
+  // whether neither the caller nor the autotuner chose it
+  static bool shapes_free(const erod_batch* b) { return unrequested(b) && b->plan.tuned_shape < 0; }
 
   constexpr int kShape256 = 2, kShape512 = 3;      // one element per thread
   constexpr int kShape128x2 = 8, kShape512x2 = 4;  // two
@@ -214,14 +215,15 @@ namespace erod {
 
   // The shape of the pieces of long rods: the one of seg_lanes lanes (and
   // seg_epl elements per thread when set), or the main shape; -2 if none.
-  // With every shape free, smaller pieces than the main tiles where those
+  // With every shape `free` (the caller requested none; the main one may be a
+  // tuned one or a trial's), smaller pieces than the main tiles where those
   // would leave CUs idle, and always for fused FP64, whose 1024-lane tiles
   // spill registers.  24 rods of 2,500 to 6,000 elements (107 / 212 / 440
   // pieces of 1024 / 512 / 256 lanes on 256 CUs), us a step: FP32-bulk 6.0 /
   // 4.4 / 4.5, FP64 21.1 / 7.7 / 8.2; 2 rods of 1,200 to 1,500: 4.6 / 3.2 / 2.7
   // and 14.8 / 6.5 / 4.5; 60 rods of 1,100 to 6,000 (206 / 391 / 803): 6.4 / 7.3
   // / 7.0 and 22.8 / 13.7 / 13.1.
-  static int piece_shape(const erod_batch* b, int main_shape, int precision) {
+  static int piece_shape(const erod_batch* b, int main_shape, int precision, bool free) {
     if (b->plan.seg_lanes > 0) {
       for (int si : {0, 1, 2, 4, 5, 3, 7, 6, 8})  // the default order of preference
         if (fused_shape_lanes(si) == b->plan.seg_lanes && (b->plan.seg_epl <= 0 || fused_shape_epl(si) == b->plan.seg_epl))
@@ -229,9 +231,7 @@ namespace erod {
       return -2;
     }
     const uint64_t halo = uint64_t(b->plan.halo);
-    if (!shapes_free(b) || !halo_fits_256(b) ||
-        (fused_shape_lanes(main_shape) != 1024 && (precision != EROD_FP64 || main_shape != kShape256)))
-      return main_shape;
+    if (!free || !halo_fits_256(b) || fused_shape_lanes(main_shape) != 1024) return main_shape;
     uint64_t pieces256 = 0, pieces512 = 0;
     for (uint64_t r = 0; r < b->n_rods; ++r)
       if (planned(b, r) && cut_rod(b, b->n_active[r], main_shape)) {
@@ -441,7 +441,8 @@ namespace erod {
     return -2;
   }
 
-  static int plan_tiles(erod_batch* b, int si, int ps, int precision) {
+  // free: the caller requested no shape
+  static int plan_tiles(erod_batch* b, int si, int ps, int precision, bool free) {
     const uint64_t cap = uint64_t(fused_shape_lanes(si));
     if (ps == -2) {
       set_error("plan_tiles: no tile shape of the requested piece lanes and elements per thread");
@@ -457,7 +458,7 @@ namespace erod {
     std::vector<uint32_t> len(b->n_rods), whole;
     std::vector<uint32_t> seg_rods;
     std::vector<Seg> segs;
-    const uint64_t wide = b->plan.seg_lanes == 0 && halo == 16 && shapes_free(b) ? wide_halo(b, si, pcap, halo) : halo;
+    const uint64_t wide = b->plan.seg_lanes == 0 && halo == 16 && free ? wide_halo(b, si, pcap, halo) : halo;
     for (uint32_t i = 0; i < b->n_rods; ++i) {
       if (!planned(b, i)) continue;
       len[i] = static_cast<uint32_t>(b->n_active[i]);
@@ -569,7 +570,8 @@ namespace erod {
                   "a rod has)");
         return EROD_ERR_UNSUPPORTED;
       }
-      const int ps = piece_shape(b, si, precision);
+      const bool free = unrequested(b);
+      const int ps = piece_shape(b, si, precision, free);
       if (pl.valid && (si != pl.main_shape || ps != pl.piece_shape)) {
         // other shapes than this plan's: the kept one comes in, this one is kept
         for (int k = 0; k < 3; ++k) std::swap(pl.g[k], pl.kept.g[k]);
@@ -578,7 +580,7 @@ namespace erod {
         std::swap(pl.valid, pl.kept.valid);
         pl.valid = pl.valid && pl.main_shape == si && pl.piece_shape == ps;
       }
-      if (!pl.valid && (rc = plan_tiles(b, si, ps, precision))) return rc;
+      if (!pl.valid && (rc = plan_tiles(b, si, ps, precision, free))) return rc;
       pl.precision = precision;
       pl.brief = brief;
     }
@@ -688,8 +690,12 @@ namespace erod {
     b->plan.lanes_per_tile = 0;
     b->plan.elements_per_thread = 0;
     b->budgets = false;  // trial launches leave the step budgets alone
-    // pieces of the requested shape, or of the main one
-    auto tuned_pieces = [&](int si) { return b->plan.seg_lanes > 0 ? piece_shape(b, si, precision) : si; };
+    // each trial's plan is the one that its shape would get once chosen, pieces
+    // and halos included (for 24 rods of 2,500 to 6,000 elements that is the
+    // untuned plan or a faster one, not launches of 16 steps over pieces of the
+    // main shape)
+    const bool free = g.lanes == 0 && g.epl == 0;
+    auto plan = [&](int si) { return plan_tiles(b, si, piece_shape(b, si, precision, free), precision, free); };
     b->plan.kept.valid = false;
     // (fused FP64 has no registers for two elements: 47 us a step on 8,192 rods
     // of 128 elements, 29 at one)
@@ -698,7 +704,7 @@ namespace erod {
     double best_t = 0.0;
     for (int si = 0; si < fused::kNShapes && rc == EROD_OK; ++si) {
       if (!shape_feasible(b, si) || !candidate(si)) continue;
-      if ((rc = plan_tiles(b, si, tuned_pieces(si), precision))) break;
+      if ((rc = plan(si))) break;
       if ((rc = fused_launch(b, precision, trial_steps, false))) break;  // warm
       if ((rc = fused_launch(b, precision, trial_steps, true))) break;
       float ms = 0.0f;
@@ -718,7 +724,7 @@ namespace erod {
         if (fused_shape_lanes(s2) >= cap || !candidate(s2)) continue;
         b->plan.split_lanes = fused_shape_lanes(s2);
         b->plan.split_epl = fused_shape_epl(s2);
-        const int prc = plan_tiles(b, best, tuned_pieces(best), precision);
+        const int prc = plan(best);
         if (prc == EROD_ERR_HIP) {  // a device failure ends the search; an infeasible shape does not
           rc = prc;
           break;
@@ -747,7 +753,7 @@ namespace erod {
     b->plan.split_epl = best_split >= 0 ? fused_shape_epl(best_split) : g.split_epl;
     g.keep_split = true;
     b->budgets = g.budgets;
-    if (rc == EROD_OK && best >= 0) rc = plan_tiles(b, best, tuned_pieces(best), precision);
+    if (rc == EROD_OK && best >= 0) rc = plan(best);
     if (rc == EROD_OK) rc = restore();
     if (rc == EROD_OK) rc = hip_check(hipStreamSynchronize(b->stream), "autotune");
     if (rc == EROD_OK && best < 0) {

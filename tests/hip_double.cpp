@@ -182,7 +182,7 @@ Error hipLaunchKernel(const void* f, Dim3 grid, Dim3 block, void** args, size_t,
   if (name.find("k_fused") != std::string::npos) {
     const int total = *static_cast<int*>(args[13]), split = *static_cast<int*>(args[14]);
     note("launch %s grid %u steps %d split %d foreign %d", name.c_str(), grid.x, total, split, foreign(args, stream->device));
-    g_clock += unit * total;
+    g_clock += unit * (total + 8);
   } else if (name.find("k_steps") != std::string::npos) {
     note("launch %s grid %u steps %d left %d own %d foreign %d", name.c_str(), grid.x, *static_cast<int*>(args[10]),
          *static_cast<int*>(args[11]), *static_cast<int*>(args[12]), foreign(args, stream->device));

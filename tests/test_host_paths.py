@@ -157,3 +157,39 @@ for precision, fast in ((FP32_BULK, b"k_fusedIfLi1ELi256E"), (FP64, b"k_fusedIdL
             blk.step_fused(n, precision)
             assert [l[1:3] for l in launches()] == [(1, 256)], (precision, lanes, n, launches())
 """)
+
+
+@pytest.mark.parametrize("lengths", ["[2500] * 12 + [6000] * 12", "[1100, 1500]", "[700] * 40 + [5000] * 3", "[1300, 30, 200, 2000]",
+                                     "[5000] * 40", "[400, 100, 512]"])
+@pytest.mark.parametrize("precision,letter", [("FP64", "d"), ("FP32_BULK", "f")])
+def test_the_autotuner_keeps_the_plan_it_timed(run, precision, letter, lengths):
+    """Whichever shape is fastest: the launches of the batch afterwards are the
+    ones its trial timed, in their number, pieces and steps, after replans too,
+    and cover the plan of an untuned batch."""
+    run("""
+T = 60
+free = block(%(lengths)s)
+free.step_fused(T, %(precision)s)
+free = launches()
+trials = []
+for shape in ("Li1ELi256E", "Li1ELi512E", "Li2ELi512E", "Li2ELi256E"):
+    blk = block(%(lengths)s)
+    D.double_fast(("k_fusedI%(letter)s" + shape).encode())
+    best = blk.autotune(%(precision)s, T)
+    seen = launches()
+    trials += seen
+    for replan in (0, 1, 2):
+        D.double_clear()
+        if replan == 1:
+            blk.set_fused_split(*blk.fused_split()[:2])
+        if replan == 2:
+            assert abs(blk.autotune(%(precision)s, T) - best) < 1e-6, shape
+            D.double_clear()
+        blk.step_fused(T, %(precision)s)
+        now = launches()
+        n = len(now)
+        assert any(seen[i:i + n] == now for i in range(len(seen))), (shape, replan, now)
+        assert abs(blk.last_kernel_ms()[0] / T - best) < 1e-6, (shape, replan)
+n = len(free)
+assert any(trials[i:i + n] == free for i in range(len(trials))), free
+""" % dict(precision=precision, letter=letter, lengths=lengths))
