@@ -689,6 +689,7 @@ int erod_set_fused_split(erod_batch* b, int lanes_per_tile, int elements_per_thr
   }
   b->plan.split_lanes = lanes_per_tile;
   b->plan.split_epl = elements_per_thread;
+  b->plan.split_tuned = false;
   b->plan.valid = false;
   b->graph_precision = -1;
   return EROD_OK;

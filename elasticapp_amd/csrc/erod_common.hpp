@@ -135,6 +135,7 @@ namespace erod {
     // optional second group: rods of at most split_lanes elements that find no
     // room beside longer rods run in tiles of that shape, in a second launch
     int split_lanes = 0, split_epl = 0;  // requested (0 = no second group)
+    bool split_tuned = false;            // by the autotuner
     // rods longer than the main tile, or than seg_lanes when it is set, run
     // as overlapping pieces of at most seg_lanes (0: the main tile's) lanes
     // with `halo` elements recomputed on each side
@@ -143,15 +144,15 @@ namespace erod {
     TileGroup g[3];
     bool valid = false;
     // where the caller leaves the shapes free they depend on the precision and
-    // on whether the call's launches are shorter than a halo: both, the main
-    // shape and pieces' shape of g, and the plan of the other calls, kept while
-    // both are in use
-    int precision = -1, main_shape = -1, piece_shape = -1;
+    // on whether the call's launches are shorter than a halo: both, the main,
+    // pieces' and second group's shapes of g, and the plan of the other calls,
+    // kept while both are in use
+    int precision = -1, main_shape = -1, piece_shape = -1, split_shape = -1;
     bool brief = false;
     struct Kept {
       TileGroup g[3];
       bool valid = false;
-      int main_shape = -1, piece_shape = -1;
+      int main_shape = -1, piece_shape = -1, split_shape = -1;
     } kept;
   };
 

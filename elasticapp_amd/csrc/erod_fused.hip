@@ -135,8 +135,8 @@ namespace erod {
   // whether neither the caller nor the autotuner chose it
   static bool shapes_free(const erod_batch* b) { return unrequested(b) && b->plan.tuned_shape < 0; }
 
-  constexpr int kShape256 = 2, kShape512 = 3;      // one element per thread
-  constexpr int kShape128x2 = 8, kShape512x2 = 4;  // two
+  constexpr int kShape128 = 1, kShape256 = 2, kShape512 = 3;  // one element per thread
+  constexpr int kShape128x2 = 8, kShape512x2 = 4;             // two
 
   // whether the second state copy that pieces need is there, or can be without
   // taking the last of the memory (or, for a server's pool, memory that its HBM
@@ -183,10 +183,15 @@ namespace erod {
   // 13.6 -> 3.5 for 20 of them, but take 1024 lanes by promise: an autotune, or
   // a request for pieces, has them faster.)
   // A shape the autotuner chose is taken again while it stays feasible (a
-  // replan after rods changed length keeps it, with its second group).
+  // replan after rods changed length keeps it, with its second group).  Tuned
+  // for FP32-bulk, 128 lanes may have two elements per thread in one wave, for
+  // which FP64 has no registers (8,192 rods of 128 elements 47 us a step, 29 at
+  // one): it takes one.
   static int default_shape(const erod_batch* b, int precision, bool brief) {
     static const int pref[] = {0, 1, 2, 4, 5, 3, 7, 6, 8};
-    if (b->plan.tuned_shape >= 0 && shape_feasible(b, b->plan.tuned_shape)) return b->plan.tuned_shape;
+    const int tuned = b->plan.tuned_shape;
+    if (tuned >= 0 && shape_feasible(b, tuned))
+      return tuned == kShape128x2 && precision == EROD_FP64 && shape_feasible(b, kShape128) ? kShape128 : tuned;
     uint64_t maxn = 0, lanes = 0;
     for (uint64_t r = 0; r < b->n_rods; ++r)
       if (planned(b, r)) {
@@ -211,6 +216,17 @@ namespace erod {
     for (int si : {5, 4, 3, 2, 1, 0, 7, 6, 8})
       if (shape_feasible(b, si)) return si;
     return -1;
+  }
+
+  // the shape a requested or tuned second group uses, or -1 (none)
+  static int split_shape(const erod_batch* b, int precision) {
+    if (b->plan.split_lanes <= 0) return -1;
+    if (b->plan.split_tuned && precision == EROD_FP64 && b->plan.split_lanes == 128) return kShape128;
+    for (int si : {0, 1, 2, 4, 5, 3, 7, 6, 8})  // the default order of preference
+      if (fused::kShapes[si].P * fused::kShapes[si].NT == b->plan.split_lanes &&
+          (b->plan.split_epl <= 0 || fused::kShapes[si].P == b->plan.split_epl))
+        return si;
+    return -2;
   }
 
   // The shape of the pieces of long rods: the one of seg_lanes lanes (and
@@ -431,16 +447,6 @@ namespace erod {
     return EROD_OK;
   }
 
-  // the shape a requested second group uses, or -1 (none requested)
-  static int split_shape(const erod_batch* b) {
-    if (b->plan.split_lanes <= 0) return -1;
-    for (int si : {0, 1, 2, 4, 5, 3, 7, 6, 8})  // the default order of preference
-      if (fused::kShapes[si].P * fused::kShapes[si].NT == b->plan.split_lanes &&
-          (b->plan.split_epl <= 0 || fused::kShapes[si].P == b->plan.split_epl))
-        return si;
-    return -2;
-  }
-
   // free: the caller requested no shape
   static int plan_tiles(erod_batch* b, int si, int ps, int precision, bool free) {
     const uint64_t cap = uint64_t(fused_shape_lanes(si));
@@ -473,7 +479,7 @@ namespace erod {
         whole.push_back(i);
       }
     }
-    const int s2 = split_shape(b);
+    const int s2 = split_shape(b, precision);
     if (s2 == -2) {
       set_error("plan_tiles: no tile shape of the requested split lanes and elements per thread");
       return EROD_ERR_INVALID;
@@ -550,6 +556,7 @@ namespace erod {
     pl.precision = precision;
     pl.main_shape = si;
     pl.piece_shape = ps;
+    pl.split_shape = s2;
     pl.valid = true;
     b->graph_precision = -1;
     return EROD_OK;
@@ -572,13 +579,16 @@ namespace erod {
       }
       const bool free = unrequested(b);
       const int ps = piece_shape(b, si, precision, free);
-      if (pl.valid && (si != pl.main_shape || ps != pl.piece_shape)) {
+      const int s2 = split_shape(b, precision);
+      const auto same = [&](const auto& p) { return p.main_shape == si && p.piece_shape == ps && p.split_shape == s2; };
+      if (pl.valid && !same(pl)) {
         // other shapes than this plan's: the kept one comes in, this one is kept
         for (int k = 0; k < 3; ++k) std::swap(pl.g[k], pl.kept.g[k]);
         std::swap(pl.main_shape, pl.kept.main_shape);
         std::swap(pl.piece_shape, pl.kept.piece_shape);
+        std::swap(pl.split_shape, pl.kept.split_shape);
         std::swap(pl.valid, pl.kept.valid);
-        pl.valid = pl.valid && pl.main_shape == si && pl.piece_shape == ps;
+        pl.valid = pl.valid && same(pl);
       }
       if (!pl.valid && (rc = plan_tiles(b, si, ps, precision, free))) return rc;
       pl.precision = precision;
@@ -697,8 +707,7 @@ namespace erod {
     const bool free = g.lanes == 0 && g.epl == 0;
     auto plan = [&](int si) { return plan_tiles(b, si, piece_shape(b, si, precision, free), precision, free); };
     b->plan.kept.valid = false;
-    // (fused FP64 has no registers for two elements: 47 us a step on 8,192 rods
-    // of 128 elements, 29 at one)
+    // (as default_shape would not take it)
     auto candidate = [&](int si) { return si != kShape128x2 || precision != EROD_FP64; };
     int best = -1;
     double best_t = 0.0;
@@ -751,6 +760,7 @@ namespace erod {
     b->plan.elements_per_thread = g.epl;
     b->plan.split_lanes = best_split >= 0 ? fused_shape_lanes(best_split) : g.split_lanes;
     b->plan.split_epl = best_split >= 0 ? fused_shape_epl(best_split) : g.split_epl;
+    b->plan.split_tuned |= best_split >= 0;
     g.keep_split = true;
     b->budgets = g.budgets;
     if (rc == EROD_OK && best >= 0) rc = plan(best);

@@ -242,6 +242,7 @@ namespace {
     p->plan.steps_per_launch = old->plan.steps_per_launch;
     p->plan.split_lanes = old->plan.split_lanes;
     p->plan.split_epl = old->plan.split_epl;
+    p->plan.split_tuned = old->plan.split_tuned;
     p->plan.seg_lanes = old->plan.seg_lanes;
     p->plan.seg_epl = old->plan.seg_epl;
     p->plan.halo = old->plan.halo;

@@ -28,6 +28,9 @@ def launches():
     return [(a[0], int(a[1]), int(a[2]), int(a[3]), int(a[4]), int(a[5])) for a in
             re.findall(r"k_fusedI([df])Li(\\d+)ELi(\\d+)ELi\\d+ELb([01])E\\S* grid (\\d+) steps (\\d+)", D.double_log().decode())]
 
+def fast(name, faster=b""):
+    D.double_fast(name, faster)
+
 def block(lengths):
     b = DeviceBlock(list(lengths))
     b.set_rod_dt(1e-5)
@@ -146,11 +149,11 @@ def test_a_tuned_plan_outlives_calls_of_another_length(run):
     """The plan an autotune leaves in place stands for calls longer and shorter
     than its trials, also where the caller had requested another shape."""
     run("""
-for precision, fast in ((FP32_BULK, b"k_fusedIfLi1ELi256E"), (FP64, b"k_fusedIdLi1ELi256E")):
+for precision, name in ((FP32_BULK, b"k_fusedIfLi1ELi256E"), (FP64, b"k_fusedIdLi1ELi256E")):
     for lanes in (0, 512):
         blk = block([200, 250, 30, 100])
         blk.set_fused_config(lanes, 0, 0)
-        D.double_fast(fast)
+        fast(name)
         blk.autotune(precision, 4)
         for n in (100, 3, 100):
             D.double_clear()
@@ -174,7 +177,7 @@ free = launches()
 trials = []
 for shape in ("Li1ELi256E", "Li1ELi512E", "Li2ELi512E", "Li2ELi256E"):
     blk = block(%(lengths)s)
-    D.double_fast(("k_fusedI%(letter)s" + shape).encode())
+    fast(("k_fusedI%(letter)s" + shape).encode())
     best = blk.autotune(%(precision)s, T)
     seen = launches()
     trials += seen
@@ -193,3 +196,34 @@ for shape in ("Li1ELi256E", "Li1ELi512E", "Li2ELi512E", "Li2ELi256E"):
 n = len(free)
 assert any(trials[i:i + n] == free for i in range(len(trials))), free
 """ % dict(precision=precision, letter=letter, lengths=lengths))
+
+
+def test_fp64_on_a_batch_tuned_for_fp32(run):
+    """FP64 has no registers for two elements per thread in one wave: it takes
+    128 lanes at one where the autotuner chose that shape for FP32-bulk, as the
+    main one or the second group's, and a caller's own request stands."""
+    run("""
+def shapes(b, precision):
+    D.double_clear()
+    b.step_fused(30, precision)
+    return {l[1:3] for l in launches()}
+blk = block([100] * 50)
+fast(b"k_fusedIfLi2ELi64E")
+blk.autotune(FP32_BULK, 20)
+for _ in range(2):
+    assert shapes(blk, FP32_BULK) == {(2, 64)} and shapes(blk, FP64) == {(1, 128)}
+    assert not _ or not log("copy device")  # (both plans are kept)
+blk.set_fused_config(128, 2, 0)
+assert shapes(blk, FP64) == {(2, 64)}
+
+fast(b"k_fusedIfLi1ELi512E", b"k_fusedIfLi2ELi64ELi0ELb0E")
+blk = block([500] * 300 + [20] * 300)
+blk.autotune(FP32_BULK, 20)
+assert blk.fused_split()[:2] == (128, 2)
+for _ in range(2):
+    assert shapes(blk, FP32_BULK) == {(1, 512), (2, 64)} and shapes(blk, FP64) == {(1, 512), (1, 128)}
+    assert not _ or not log("copy device")
+blk = block([500] * 300 + [20] * 300)
+blk.set_fused_split(128, 2)
+assert (2, 64) in shapes(blk, FP64)
+""")
