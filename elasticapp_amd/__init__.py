@@ -340,7 +340,9 @@ class DeviceBlock:
         _check(_LIB.erod_set_fused_pieces(self._h, int(lanes_per_tile), int(elements_per_thread), int(halo)))
 
     def fused_pieces(self):
-        """(lanes, elements per thread, halo, tiles, pieces) of the current plan's pieces."""
+        """(lanes, elements per thread, halo, tiles, pieces) of the current plan's
+        pieces; the halo is the one requested (16 if free, also where the plan
+        widens it)."""
         a, b, h, t, p = ctypes.c_int(), ctypes.c_int(), ctypes.c_int(), ctypes.c_uint64(), ctypes.c_uint64()
         _check(_LIB.erod_get_fused_pieces(self._h, ctypes.byref(a), ctypes.byref(b), ctypes.byref(h), ctypes.byref(t),
                                           ctypes.byref(p)))

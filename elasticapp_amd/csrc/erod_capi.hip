@@ -712,6 +712,7 @@ int erod_set_fused_pieces(erod_batch* b, int lanes_per_tile, int elements_per_th
   b->plan.seg_lanes = lanes_per_tile;
   b->plan.seg_epl = elements_per_thread;
   b->plan.halo = halo ? halo : 16;
+  b->plan.halo_set = halo != 0;
   b->plan.valid = false;
   b->graph_precision = -1;
   return EROD_OK;

@@ -138,8 +138,10 @@ namespace erod {
     bool split_tuned = false;            // by the autotuner
     // rods longer than the main tile, or than seg_lanes when it is set, run
     // as overlapping pieces of at most seg_lanes (0: the main tile's) lanes
-    // with `halo` elements recomputed on each side
+    // with `halo` elements recomputed on each side (more where halo_set, the
+    // caller's request, leaves that free)
     int seg_lanes = 0, seg_epl = 0, halo = 16;
+    bool halo_set = false;
     // groups: 0 main, 1 second (short rods), 2 pieces of long rods
     TileGroup g[3];
     bool valid = false;

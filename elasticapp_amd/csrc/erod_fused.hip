@@ -464,7 +464,7 @@ namespace erod {
     std::vector<uint32_t> len(b->n_rods), whole;
     std::vector<uint32_t> seg_rods;
     std::vector<Seg> segs;
-    const uint64_t wide = b->plan.seg_lanes == 0 && halo == 16 && free ? wide_halo(b, si, pcap, halo) : halo;
+    const uint64_t wide = b->plan.seg_lanes == 0 && !b->plan.halo_set && free ? wide_halo(b, si, pcap, halo) : halo;
     for (uint32_t i = 0; i < b->n_rods; ++i) {
       if (!planned(b, i)) continue;
       len[i] = static_cast<uint32_t>(b->n_active[i]);
@@ -547,7 +547,7 @@ namespace erod {
     gs.n_segs = segs.size();
     gs.n_seg_rods = seg_rods.size();
     // FP32-bulk's merged half steps end every halo / 2 steps, wherever launches
-    // end; a launch holds two such runs.  13 launches per 100 steps (halo 16)
+    // end; a launch holds two such runs (three for a halo of 3, more in a wide one).  13 launches per 100 steps (halo 16)
     // became 7: 24 rods of 2,500 to 6,000 elements 6.05 -> 5.08 us a step
     // (FP32-bulk), 2,048 ragged rods 29.6 -> 28.0 (FP64, long rods in pieces)
     gs.run_steps = int(halo / 2);

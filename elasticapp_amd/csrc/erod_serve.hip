@@ -246,6 +246,7 @@ namespace {
     p->plan.seg_lanes = old->plan.seg_lanes;
     p->plan.seg_epl = old->plan.seg_epl;
     p->plan.halo = old->plan.halo;
+    p->plan.halo_set = old->plan.halo_set;
     p->plan.tuned_shape = old->plan.tuned_shape;
     // and so does the re-orthonormalisation schedule, at its phase
     p->reortho_every = old->reortho_every;

@@ -181,8 +181,9 @@ int erod_set_rod_time(erod_batch* b, const double* time_per_rod);
  * otherwise; FP32-bulk batches that fill the device take two elements per
  * thread in 128 lanes for rods of up to 128 elements, in 512 for rods of up to
  * 256; small FP64 batches whose longest rod has 257 to 512 elements take 256
- * lanes, but for calls of launches shorter than 16 steps); rods longer than the tile run as pieces
- * (erod_set_fused_pieces).  Results do not depend on the shape. */
+ * lanes, but for calls of launches shorter than 16 steps); rods longer than
+ * the tile run as pieces (erod_set_fused_pieces).  Results do not depend on the
+ * shape, bit for bit; FP32-bulk's not on one that leaves the same rods whole. */
 int erod_set_fused_config(erod_batch* b, int lanes_per_tile, int elements_per_thread, int steps_per_launch);
 int erod_get_fused_config(const erod_batch* b, int* lanes_per_tile, int* elements_per_thread, int* steps_per_launch);
 /* A second group of tiles: a rod of at most lanes_per_tile elements that finds
@@ -195,19 +196,24 @@ int erod_get_fused_config(const erod_batch* b, int* lanes_per_tile, int* element
 int erod_set_fused_split(erod_batch* b, int lanes_per_tile, int elements_per_thread);
 int erod_get_fused_split(const erod_batch* b, int* lanes_per_tile, int* elements_per_thread, uint64_t* tiles);
 /* Rods longer than the main tile, or longer than lanes_per_tile when it is
- * not 0, run as pieces in tiles of that shape (0: the main shape, or, when no
- * shape was requested or tuned, smaller tiles where those leave fewer compute
- * units idle, and 256 lanes for FP64; elements_per_thread 0 = either): each
- * piece owns a part of its rod and
- * recomputes `halo` elements (0 = 16, at least 2) of each neighbouring piece
+ * not 0, run as pieces in tiles of that shape (0: the main shape, or, beside
+ * main tiles of 1024 lanes when no shape was requested, smaller tiles where
+ * those leave fewer compute units idle, and 256 lanes for FP64;
+ * elements_per_thread 0 = either): each piece owns a part of its rod and
+ * recomputes `halo` elements (0 = free, at least 2) of each neighbouring piece
  * from the state they had when the launch began, so that pieces need no
- * exchange within a launch; a launch over pieces then takes at most halo (or
- * halo - 1, if odd) steps, and the pieces' group is launched as often as
- * needed.  (Where neither shape nor halo was requested, halos widen to up to 64
- * elements while every piece has a compute unit of its own.)  Results do not depend on the cut (bitwise).  For rods longer than any tile (the
- * reference's blocks emplace rods of any length, Block.hpp:568-611) and for
- * fused FP64, whose long-rod tiles spill registers.  The getter reports the
- * pieces' shape, halo, tiles and pieces in the current plan (0 if none). */
+ * exchange within a launch; a launch over pieces then takes at most halo
+ * (halo - 1, if odd and above 3) steps, and the pieces' group is launched as
+ * often as needed.  A free halo is 16; where no shape was requested either, it
+ * widens to up to 64 elements while every piece has a compute unit of its own.
+ * FP64 results do not depend on the cut, bit for bit.  FP32-bulk's depend on
+ * whether a rod is cut and on the halo requested (16 if free), not on the
+ * pieces' shape or on widening: the half steps that it merges inside a launch
+ * end every halo / 2 steps of a rod that is cut.  For rods longer than any tile
+ * (the reference's blocks emplace rods of any length, Block.hpp:568-611) and
+ * for fused FP64, whose long-rod tiles spill registers.  The getter reports
+ * the pieces' shape, tiles and pieces in the current plan (0 if none), and the
+ * halo requested (16 if free, whether or not the plan widens it). */
 int erod_set_fused_pieces(erod_batch* b, int lanes_per_tile, int elements_per_thread, int halo);
 int erod_get_fused_pieces(const erod_batch* b, int* lanes_per_tile, int* elements_per_thread, int* halo,
                           uint64_t* tiles, uint64_t* pieces);

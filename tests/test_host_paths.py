@@ -227,3 +227,24 @@ blk = block([500] * 300 + [20] * 300)
 blk.set_fused_split(128, 2)
 assert (2, 64) in shapes(blk, FP64)
 """)
+
+
+def test_a_requested_halo_is_not_widened(run):
+    """A halo of 16 that the caller asked for stays 16, in any precision and
+    after an autotune; one left free widens, and is free again with 0."""
+    run("""
+for precision, name in ((FP64, b"k_fusedIdLi1ELi256E"), (FP32_BULK, b"k_fusedIfLi1ELi256E")):
+    fast(name)
+    for tuned in (0, 1):
+        blk = block([1500, 2000])
+        counts = []
+        for halo in (0, 16, 0):
+            blk.set_fused_pieces(0, 0, halo)
+            if tuned:
+                blk.autotune(precision, 64)
+            D.double_clear()
+            blk.step_fused(64, precision)
+            counts.append((max(l[5] for l in launches()), blk.fused_pieces()[4]))
+        assert [c[0] for c in counts] == [64, 16, 64], counts
+        assert counts[0] == counts[2] and counts[0][1] > counts[1][1], counts
+""")
