@@ -851,7 +851,7 @@ namespace erod {
     uint64_t launches = (n + most - 1) / most;
     if (!one) launches += launches & 1;
     for (uint64_t i = 0; i < launches; ++i) {
-      const int s = static_cast<int>((i + 1) * n / launches - i * n / launches);
+      const int s = static_cast<int>(n / launches + (i < n % launches ? 1 : 0));
       const int left = one ? 0 : s, own = one ? static_cast<int>(N) : kThreads - 1 - 2 * s;
       const bool odd = !one && (i & 1);
       hipLaunchKernelGGL(k_steps, dim3(static_cast<unsigned>((N + own - 1) / own)), dim3(kThreads), 0, b->stream,

@@ -12,6 +12,7 @@
 #include <map>
 #include <mutex>
 #include <string>
+#include <utility>
 
 namespace {
   using Error = int;
@@ -33,6 +34,8 @@ namespace {
   std::map<const void*, std::string> g_kernels;
   size_t g_capacity = size_t(64) << 30, g_live[2] = {};
   double g_clock = 0.0;
+  long g_left = -1;
+  Error g_last = kOk;
   std::string g_log, g_fast[2];
   thread_local int t_device = 0;
   struct Call {
@@ -106,6 +109,7 @@ void double_fast(const char* name, const char* faster) {
 }
 const char* double_log() { return g_log.c_str(); }
 void double_clear() { g_log.clear(); }
+void double_fail_after(long n) { g_left = n; }  // launches until one is refused
 int double_set_device(int d) { return t_device = d, 0; }
 
 // ---- the runtime's calls
@@ -113,7 +117,7 @@ Error hipGetDeviceCount(int* n) { return *n = 2, kOk; }
 Error hipGetDevice(int* d) { return *d = t_device, kOk; }
 Error hipSetDevice(int d) { return t_device = d, kOk; }
 Error hipDeviceGetAttribute(int* v, int, int) { return *v = 256, kOk; }  // (only the compute units are asked for)
-Error hipGetLastError() { return kOk; }
+Error hipGetLastError() { return std::exchange(g_last, kOk); }
 const char* hipGetErrorString(Error e) { return e == kNoMemory ? "out of memory" : "error"; }
 
 Error hipMalloc(void** p, size_t bytes) {
@@ -181,6 +185,7 @@ Error hipGraphLaunch(void*, Handle*) {
 }
 
 Error hipLaunchKernel(const void* f, Dim3 grid, Dim3 block, void** args, size_t, Handle* stream) {
+  if (g_left >= 0 && g_left-- == 0) return g_last = kInvalid;
   const std::string& name = g_kernels[f];
   double unit = 1.0;
   for (int i = 0; i < 2; ++i)

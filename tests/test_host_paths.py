@@ -248,3 +248,20 @@ for precision, name in ((FP64, b"k_fusedIdLi1ELi256E"), (FP32_BULK, b"k_fusedIfL
         assert [c[0] for c in counts] == [64, 16, 64], counts
         assert counts[0] == counts[2] and counts[0][1] > counts[1][1], counts
 """)
+
+
+@pytest.mark.parametrize("n", ["25", "26", "101", "2**31 + 5", "2**40 + 7", "2**62 + 3"])
+def test_launches_of_any_number_of_steps(run, n):
+    """However many op-by-op steps one call asks for, each launch takes 12 of
+    them at most and fits its workgroups."""
+    run("""
+blk = block([400, 30])
+D.double_fail_after(ctypes.c_long(100))
+try:
+    blk.step(1e-9, %(n)s)
+except ea.ErodError:
+    pass
+steps = [tuple(int(x) for x in re.search(r"steps (-?\\d+) left (-?\\d+) own (-?\\d+)", l).groups()) for l in log("k_steps")]
+assert steps and all(1 <= s <= 12 and left == s and own == 255 - 2 * s for s, left, own in steps), steps
+assert len(steps) %% 2 == 0 and (len(steps) == 100 or sum(s[0] for s in steps) == %(n)s - 1), steps
+""" % dict(n=n))
