@@ -316,6 +316,10 @@ namespace erod {
   void free_transfer_buffers(erod_batch* b);
   // device copy of whole rods between batches (admission of a request)
   int serve_copy_rods(erod_batch* dst, const erod_batch* src, const std::vector<CopyPair>& pairs);
+  // whether the second state copy that a faster path would take is there, or can
+  // be without taking the last of the memory (or, for a server's pool, memory
+  // that its HBM budget doesn't count)
+  bool shadow_fits(const erod_batch* b);
   int fused_shape_lanes(int shape);
   int fused_shape_epl(int shape);
   int sync_rods(erod_batch* b);

@@ -138,10 +138,7 @@ namespace erod {
   constexpr int kShape128 = 1, kShape256 = 2, kShape512 = 3;  // one element per thread
   constexpr int kShape128x2 = 8, kShape512x2 = 4;             // two
 
-  // whether the second state copy that pieces need is there, or can be without
-  // taking the last of the memory (or, for a server's pool, memory that its HBM
-  // budget doesn't count)
-  static bool shadow_fits(const erod_batch* b) {
+  bool shadow_fits(const erod_batch* b) {
     if (b->d_shadow[3]) return true;
     if (b->pool) return false;
     size_t free = 0, total = 0;

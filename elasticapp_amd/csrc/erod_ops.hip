@@ -820,11 +820,17 @@ namespace erod {
   static bool steps_buffers(erod_batch* b) {
     const OnDevice here(b->device);
     static const int fields[4] = {EROD_POSITION, EROD_VELOCITY, EROD_DIRECTOR, EROD_ANGULAR_VELOCITY};
-    bool ok = true;
-    if (b->E + 1 > kThreads)
+    const bool two = b->E + 1 > kThreads;
+    bool ok = !two || shadow_fits(b);
+    if (two && ok)
       for (int i = 0; i < 4 && ok; ++i)
         if (!b->d_shadow[i])
           ok = hipMalloc(&b->d_shadow[i], sizeof(double) * field_info(fields[i]).ncomp * b->field_slots(fields[i])) == hipSuccess;
+    if (two && !ok)  // (no part of a copy that is of no use)
+      for (double*& p : b->d_shadow) {
+        (void)hipFree(p);
+        p = nullptr;
+      }
     if (ok && !b->d_slot_rods && (b->has_clamps || b->has_forces)) {
       ok = hipMalloc(&b->d_slot_rods, sizeof(uint32_t) * (b->E + 1)) == hipSuccess;
       if (ok)

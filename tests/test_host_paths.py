@@ -265,3 +265,18 @@ steps = [tuple(int(x) for x in re.search(r"steps (-?\\d+) left (-?\\d+) own (-?\
 assert steps and all(1 <= s <= 12 and left == s and own == 255 - 2 * s for s, left, own in steps), steps
 assert len(steps) %% 2 == 0 and (len(steps) == 100 or sum(s[0] for s in steps) == %(n)s - 1), steps
 """ % dict(n=n))
+
+
+@pytest.mark.parametrize("room,several", [(1 << 20, False), (4 << 20, False), (10 << 20, False), (64 << 20, True)])
+def test_op_by_op_steps_leave_memory_to_others(run, room, several):
+    """The second copy of the state is taken where the device has plenty of room
+    for it; otherwise every step goes call by call, and nothing is kept."""
+    run("""
+blk = block([40000, 30])           # a copy of 5.8 MB
+before = D.double_live(0)
+D.double_capacity(ctypes.c_size_t(before + %d))
+blk.step(1e-5, 5)
+assert bool(log("k_steps")) == %s
+assert len(log("k_kinematic")) == (2 if %s else 10)
+assert (D.double_live(0) > before) == %s
+""" % (room, several, several, several))
