@@ -152,6 +152,30 @@ namespace erod {
   // whether pieces of 256 lanes leave a part of 64 elements between their halos
   static bool halo_fits_256(const erod_batch* b) { return 2 * b->plan.halo + 64 <= 256; }
 
+  // the longest rod and the elements of those that the plan takes
+  struct Extent {
+    uint64_t longest = 0, lanes = 0;
+  };
+  static Extent extent(const erod_batch* b) {
+    Extent e;
+    for (uint64_t r = 0; r < b->n_rods; ++r)
+      if (planned(b, r)) {
+        e.longest = std::max<uint64_t>(e.longest, b->n_active[r]);
+        e.lanes += b->n_active[r];
+      }
+    return e;
+  }
+
+  // Few FP64 rods of up to 257 to 512 elements, which run as pieces in 256 lanes
+  // (see default_shape) where the caller leaves shapes free: the halo has to
+  // leave the pieces room, and to pay for their launches (100 steps of 20 rods
+  // of 400 elements, us a step: 4.1 whole; 5.4, 4.6, 4.2, 3.8, 3.6 and 2.9 with a
+  // halo of 2, 3, 4, 6, 8 and 16).
+  static bool few_in_256(const erod_batch* b, const Extent& e, int precision) {
+    return precision == EROD_FP64 && b->plan.seg_lanes == 0 && b->plan.halo >= 6 && halo_fits_256(b) && e.longest > 256 &&
+           e.longest <= 512 && e.lanes <= 32 * uint64_t(b->cus);
+  }
+
   // Default shape without measurement: the smallest capacity that holds the
   // longest rod; one element per thread up to 256 lanes, two elements per
   // thread for 1024 lanes; rods longer than 1024 elements run as pieces.  (Four
@@ -174,9 +198,9 @@ namespace erod {
   // 301: 4.6 -> 3.4 us a step; 100 of up to 512, over the line: 4.6 and 4.8).
   // Not for calls whose launches are shorter than a halo, each of which passes
   // over the state twice more (calls on one rod of 300, us: 1 step 16 whole and
-  // 25 in pieces, 8 steps 44 and 44, 16 steps 75 and 63, 100 steps 402 and 274).  Results are the
-  // same, bit by bit; FP32-bulk's depend on where a launch ends, so its rods
-  // stay whole.  (Batches with rods of 513 to 1,024 elements would gain more,
+  // 25 in pieces, 8 steps 44 and 44, 16 steps 75 and 63, 100 steps 402 and 274).
+  // Results are the same, bit by bit; FP32-bulk's depend on where a launch ends,
+  // so its rods stay whole.  (Batches with rods of 513 to 1,024 elements would gain more,
   // 13.6 -> 3.5 for 20 of them, but take 1024 lanes by promise: an autotune, or
   // a request for pieces, has them faster.)
   // A shape the autotuner chose is taken again while it stays feasible (a
@@ -189,15 +213,9 @@ namespace erod {
     const int tuned = b->plan.tuned_shape;
     if (tuned >= 0 && shape_feasible(b, tuned))
       return tuned == kShape128x2 && precision == EROD_FP64 && shape_feasible(b, kShape128) ? kShape128 : tuned;
-    uint64_t maxn = 0, lanes = 0;
-    for (uint64_t r = 0; r < b->n_rods; ++r)
-      if (planned(b, r)) {
-        maxn = std::max<uint64_t>(maxn, b->n_active[r]);
-        lanes += b->n_active[r];
-      }
-    if (precision == EROD_FP64 && shapes_free(b) && b->plan.seg_lanes == 0 && !brief && halo_fits_256(b) && maxn > 256 &&
-        maxn <= 512 && lanes <= 32 * uint64_t(b->cus) && shadow_fits(b))
-      return kShape256;
+    const Extent e = extent(b);
+    const uint64_t maxn = e.longest, lanes = e.lanes;
+    if (shapes_free(b) && !brief && few_in_256(b, e, precision) && shadow_fits(b)) return kShape256;
     for (int si : pref)
       if (uint64_t(fused_shape_lanes(si)) >= maxn && shape_feasible(b, si)) {
         const bool two = fused_shape_lanes(si) == 512 && fused_shape_epl(si) == 2;
@@ -566,7 +584,7 @@ namespace erod {
     FusedPlan& pl = b->plan;
     if (!pl.valid) pl.kept.valid = false;  // the rods changed: so did its
     // (the calls' lengths decide on free shapes only)
-    const bool brief = precision == EROD_FP64 && shapes_free(b) && launch < uint64_t(pl.halo);
+    const bool brief = precision == EROD_FP64 && shapes_free(b) && launch < uint64_t(std::max(pl.halo, 16));
     if (!pl.valid || pl.precision != precision || pl.brief != brief) {
       const int si = default_shape(b, precision, brief);
       if (si < 0) {

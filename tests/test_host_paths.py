@@ -87,6 +87,23 @@ assert D.double_live(0) == 0 and D.double_live(1) == 0
 """)
 
 
+@pytest.mark.parametrize("halo,pieces", [(2, 0), (3, 0), (5, 0), (6, 1), (8, 1), (16, 1), (32, 1)])
+def test_small_fp64_batches_with_a_short_halo(run, halo, pieces):
+    """FP64 rods of 257 to 512 elements take pieces of 256 lanes only with a halo
+    whose launches pay for them; with a shorter one they run whole, in 512, a
+    call in one launch.  Calls of fewer than 16 steps run whole with any."""
+    run("""
+blk = block([300, 400, 20])
+blk.set_fused_pieces(0, 0, %d)
+blk.step_fused(100, FP64)
+assert any(l[3] for l in launches()) == %d and {l[1:3] for l in launches()} == {(1, 256 if %d else 512)}, launches()
+assert %d or len(launches()) == 1
+D.double_clear()
+blk.step_fused(15, FP64)
+assert [l[1:4] for l in launches()] == [(1, 512, 0)]
+""" % (halo, pieces, pieces, pieces))
+
+
 @pytest.mark.parametrize("halo,pieces", [(0, 1), (96, 1), (97, 0), (100, 0), (127, 0), (128, 0), (200, 0)])
 def test_small_fp64_batches_with_a_long_halo(run, halo, pieces):
     """FP64 rods of 257 to 512 elements take pieces of 256 lanes only with a halo
