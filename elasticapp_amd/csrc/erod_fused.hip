@@ -407,6 +407,15 @@ namespace erod {
     }
   }
 
+  // a rod of n elements that one piece holds
+  static Seg whole_piece(uint32_t rod, uint32_t n) {
+    Seg sg{};
+    sg.rod = rod;
+    sg.n = sg.w1 = n;
+    sg.ends = kSegFirst | kSegLast;
+    return sg;
+  }
+
   // The halo of the pieces where the caller left their shape free: as wide as
   // leaves every piece a CU of its own (beside the whole rods' tiles), up to
   // 64, a launch taking as many steps.  Until then wider halos cost no time,
@@ -480,6 +489,14 @@ namespace erod {
     std::vector<uint32_t> seg_rods;
     std::vector<Seg> segs;
     const uint64_t wide = b->plan.seg_lanes == 0 && !b->plan.halo_set && free ? wide_halo(b, si, pcap, halo) : halo;
+    // Few FP64 rods in 256 lanes: those that need no cut go in the pieces' group
+    // too, each as one piece.  In a group of their own they would need a
+    // hardware queue of their own: 61 rods of up to 301 elements take 3.5 us a
+    // step in two groups on two queues and 6.2 where the batch's two streams
+    // share one, which is the runtime's choice (whole in 512 lanes 4.6).
+    const bool one_group = free && si == kShape256 && ps == si && b->plan.split_lanes == 0 &&
+                           few_in_256(b, extent(b), precision);
+    uint64_t uncut = 0;
     for (uint32_t i = 0; i < b->n_rods; ++i) {
       if (!planned(b, i)) continue;
       len[i] = static_cast<uint32_t>(b->n_active[i]);
@@ -490,6 +507,10 @@ namespace erod {
         }
         seg_rods.push_back(i);
         cut(i, b->n_active[i], pcap, wide, segs);
+      } else if (one_group) {
+        seg_rods.push_back(i);
+        segs.push_back(whole_piece(i, len[i]));
+        ++uncut;
       } else {
         whole.push_back(i);
       }
@@ -559,7 +580,8 @@ namespace erod {
       pl.g[k].shape = pks[k]->tiles.empty() ? -1 : shapes[k];
       pl.g[k].max_steps = 0;
     }
-    gs.n_segs = segs.size();
+    if (uncut) pl.g[0].shape = si;  // (their tiles are the pieces')
+    gs.n_segs = segs.size() - uncut;
     gs.n_seg_rods = seg_rods.size();
     // FP32-bulk's merged half steps end every halo / 2 steps, wherever launches
     // end; a launch holds two such runs (three for a halo of 3, more in a wide one).  13 launches per 100 steps (halo 16)

@@ -71,7 +71,7 @@ D.double_set_device(1)
 blk.step(1e-5, 30)                # second copy of the state
 blk.get_field("Position")         # pinned stage
 blk.step_fused(20, FP64)          # pieces: second copy, plan
-assert log("k_steps") and len(launches()) > 1
+assert log("k_steps") and any(l[3] for l in launches())
 assert all(l.endswith("foreign 0") for l in log("foreign")), log("foreign")
 big = block([70000])              # on device 1
 D.double_set_device(0)
@@ -102,6 +102,21 @@ D.double_clear()
 blk.step_fused(15, FP64)
 assert [l[1:4] for l in launches()] == [(1, 512, 0)]
 """ % (halo, pieces, pieces, pieces))
+
+
+@pytest.mark.parametrize("lengths", ["[300, 400, 20]", "[3, 301] + [10] * 59", "[512] + [2] * 200"])
+def test_small_fp64_batches_need_one_queue(run, lengths):
+    """Rods that need no cut beside FP64 rods of 257 to 512 elements are no group
+    of their own: two groups run side by side only where the runtime gives the
+    batch's two streams two hardware queues, and take their sum elsewhere."""
+    run("""
+blk = block(%s)
+blk.step_fused(100, FP64)
+steps = [l[5] for l in launches()]
+assert {l[3] for l in launches()} == {1} and sum(steps) == 100, launches()
+assert blk.fused_config()[:2] == (256, 1) and blk.fused_pieces()[0] == 256
+assert blk.fused_pieces()[4] == sum(max(2, -(-n // 128)) for n in blk.n_elems if n > 256)  # (halos of 64)
+""" % lengths)
 
 
 @pytest.mark.parametrize("halo,pieces", [(0, 1), (96, 1), (97, 0), (100, 0), (127, 0), (128, 0), (200, 0)])
