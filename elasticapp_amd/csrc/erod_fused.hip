@@ -744,8 +744,18 @@ namespace erod {
     const bool free = g.lanes == 0 && g.epl == 0;
     auto plan = [&](int si) { return plan_tiles(b, si, piece_shape(b, si, precision, free), precision, free); };
     b->plan.kept.valid = false;
-    // (as default_shape would not take it)
-    auto candidate = [&](int si) { return si != kShape128x2 || precision != EROD_FP64; };
+    // FP64 has no registers for two elements per thread in one wave (see
+    // default_shape).  FP32-bulk rounds a rod that is cut by its halo: where 512
+    // lanes hold every rod, shapes that cut some are not tried, so that a tuned
+    // batch returns what an untuned one does, and not what the trials' times
+    // happen to decide.  (Pieces with wide halos would be faster: passes of 11
+    // rods of 105 to 258 elements 1.09 ms against 1.22, of 15 rods of 25 to 314
+    // 0.65 against 0.73.  With longer rods, beside which whole ones run in
+    // 1024 lanes, 2.9 against 4.3 for 70 of 44 to 718, they are tried.)
+    const uint64_t longest = extent(b).longest;
+    const bool keep_whole = precision != EROD_FP64 && b->plan.seg_lanes == 0 && longest <= 512;
+    auto has_registers = [&](int si) { return si != kShape128x2 || precision != EROD_FP64; };
+    auto candidate = [&](int si) { return has_registers(si) && (!keep_whole || uint64_t(fused_shape_lanes(si)) >= longest); };
     int best = -1;
     double best_t = 0.0;
     for (int si = 0; si < fused::kNShapes && rc == EROD_OK; ++si) {
@@ -767,7 +777,7 @@ namespace erod {
     if (rc == EROD_OK && best >= 0 && g.split_lanes == 0) {
       const int cap = fused_shape_lanes(best);
       for (int s2 = 0; s2 < fused::kNShapes && rc == EROD_OK; ++s2) {
-        if (fused_shape_lanes(s2) >= cap || !candidate(s2)) continue;
+        if (fused_shape_lanes(s2) >= cap || !has_registers(s2)) continue;
         b->plan.split_lanes = fused_shape_lanes(s2);
         b->plan.split_epl = fused_shape_epl(s2);
         const int prc = plan(best);

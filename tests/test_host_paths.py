@@ -230,6 +230,31 @@ assert any(trials[i:i + n] == free for i in range(len(trials))), free
 """ % dict(precision=precision, letter=letter, lengths=lengths))
 
 
+@pytest.mark.parametrize("lengths,whole", [("[105, 258, 130, 200] * 3", 1), ("[40] * 20 + [10]", 1), ("[3, 512]", 1),
+                                           ("[3, 513]", 0), ("[700] * 4 + [5000] * 3", 0)])
+def test_a_tuned_fp32_batch_keeps_its_rods_whole(run, lengths, whole):
+    """FP32-bulk rounds a rod that is cut by its halo, so where 512 lanes hold
+    every rod none is cut, of whatever shape the trials were fastest.  A caller
+    that asks for pieces has them, and FP64, the same bits either way, has any."""
+    run("""
+T, cut = 60, set()
+def tuned(precision, shape, lanes=0):
+    blk = block(%(lengths)s)
+    blk.set_fused_pieces(lanes, 0, 0)
+    fast(shape)
+    blk.autotune(precision, T)
+    D.double_clear()
+    blk.step_fused(T, precision)
+    return any(l[3] for l in launches())
+for shape in (b"Li1ELi64E", b"Li1ELi128E", b"Li1ELi256E", b"Li1ELi512E", b"Li2ELi64E", b"Li2ELi256E", b"Li2ELi512E"):
+    cut.add(tuned(FP32_BULK, b"k_fusedIf" + shape))
+assert (cut == {False}) == %(whole)d, cut
+if max(block(%(lengths)s).n_elems) > 64:
+    assert tuned(FP32_BULK, b"k_fusedIfLi1ELi64E", 64)
+    assert tuned(FP64, b"k_fusedIdLi1ELi64E")
+""" % dict(lengths=lengths, whole=whole))
+
+
 def test_fp64_on_a_batch_tuned_for_fp32(run):
     """FP64 has no registers for two elements per thread in one wave: it takes
     128 lanes at one where the autotuner chose that shape for FP32-bulk, as the
