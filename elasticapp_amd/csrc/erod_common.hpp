@@ -147,13 +147,13 @@ namespace erod {
     bool valid = false;
     // where the caller leaves the shapes free they depend on the precision and
     // on whether the call's launches are shorter than a halo: both, the main,
-    // pieces' and second group's shapes of g, and the plan of the other calls,
-    // kept while both are in use
+    // pieces' and second group's shapes of g, whether rods that need no cut are
+    // pieces too, and the plan of the other calls, kept while both are in use
     int precision = -1, main_shape = -1, piece_shape = -1, split_shape = -1;
-    bool brief = false;
+    bool one_group = false, brief = false;
     struct Kept {
       TileGroup g[3];
-      bool valid = false;
+      bool valid = false, one_group = false;
       int main_shape = -1, piece_shape = -1, split_shape = -1;
     } kept;
   };

@@ -471,6 +471,16 @@ namespace erod {
     return EROD_OK;
   }
 
+  // Few FP64 rods in 256 lanes: those that need no cut go in the pieces' group
+  // too, each as one piece.  In a group of their own they would need a hardware
+  // queue of their own: 61 rods of up to 301 elements take 3.5 us a step in two
+  // groups on two queues and 6.2 where the batch's two streams share one, which
+  // is the runtime's choice (whole in 512 lanes 4.6).  Not FP32-bulk's, which
+  // rounds a piece by its halo.
+  static bool one_group(const erod_batch* b, int si, int ps, int precision, bool free) {
+    return free && si == kShape256 && ps == si && b->plan.split_lanes == 0 && few_in_256(b, extent(b), precision);
+  }
+
   // free: the caller requested no shape
   static int plan_tiles(erod_batch* b, int si, int ps, int precision, bool free) {
     const uint64_t cap = uint64_t(fused_shape_lanes(si));
@@ -489,13 +499,7 @@ namespace erod {
     std::vector<uint32_t> seg_rods;
     std::vector<Seg> segs;
     const uint64_t wide = b->plan.seg_lanes == 0 && !b->plan.halo_set && free ? wide_halo(b, si, pcap, halo) : halo;
-    // Few FP64 rods in 256 lanes: those that need no cut go in the pieces' group
-    // too, each as one piece.  In a group of their own they would need a
-    // hardware queue of their own: 61 rods of up to 301 elements take 3.5 us a
-    // step in two groups on two queues and 6.2 where the batch's two streams
-    // share one, which is the runtime's choice (whole in 512 lanes 4.6).
-    const bool one_group = free && si == kShape256 && ps == si && b->plan.split_lanes == 0 &&
-                           few_in_256(b, extent(b), precision);
+    const bool one = one_group(b, si, ps, precision, free);
     uint64_t uncut = 0;
     for (uint32_t i = 0; i < b->n_rods; ++i) {
       if (!planned(b, i)) continue;
@@ -507,7 +511,7 @@ namespace erod {
         }
         seg_rods.push_back(i);
         cut(i, b->n_active[i], pcap, wide, segs);
-      } else if (one_group) {
+      } else if (one) {
         seg_rods.push_back(i);
         segs.push_back(whole_piece(i, len[i]));
         ++uncut;
@@ -594,6 +598,7 @@ namespace erod {
     pl.main_shape = si;
     pl.piece_shape = ps;
     pl.split_shape = s2;
+    pl.one_group = one;
     pl.valid = true;
     b->graph_precision = -1;
     return EROD_OK;
@@ -617,13 +622,17 @@ namespace erod {
       const bool free = unrequested(b);
       const int ps = piece_shape(b, si, precision, free);
       const int s2 = split_shape(b, precision);
-      const auto same = [&](const auto& p) { return p.main_shape == si && p.piece_shape == ps && p.split_shape == s2; };
+      const bool one = one_group(b, si, ps, precision, free);
+      const auto same = [&](const auto& p) {
+        return p.main_shape == si && p.piece_shape == ps && p.split_shape == s2 && p.one_group == one;
+      };
       if (pl.valid && !same(pl)) {
         // other shapes than this plan's: the kept one comes in, this one is kept
         for (int k = 0; k < 3; ++k) std::swap(pl.g[k], pl.kept.g[k]);
         std::swap(pl.main_shape, pl.kept.main_shape);
         std::swap(pl.piece_shape, pl.kept.piece_shape);
         std::swap(pl.split_shape, pl.kept.split_shape);
+        std::swap(pl.one_group, pl.kept.one_group);
         std::swap(pl.valid, pl.kept.valid);
         pl.valid = pl.valid && same(pl);
       }

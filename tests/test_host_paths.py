@@ -286,6 +286,32 @@ assert (2, 64) in shapes(blk, FP64)
 """)
 
 
+def test_fp32_on_a_batch_tuned_for_fp64(run):
+    """FP32-bulk rounds a rod that runs as a piece by its halo: which rods do is
+    the same whether the FP64 call that made the plan came before or after."""
+    run("""
+def tuned():
+    blk = block([300, 400, 20, 250])
+    fast(b"k_fusedIdLi1ELi256E")
+    blk.autotune(FP64, 100)
+    return blk
+def plan(blk, precision):
+    D.double_clear()
+    blk.step_fused(100, precision)
+    return sorted(set(l[1:5] for l in launches()))
+blk = tuned()
+blk.set_fused_split(0, 0)          # (plans are made anew)
+first = plan(blk, FP32_BULK)
+assert {l[2] for l in first} == {0, 1}, first
+both = plan(blk, FP64)
+assert {l[2] for l in both} == {1}, both
+blk = tuned()
+for _ in range(2):
+    assert plan(blk, FP64) == both and plan(blk, FP32_BULK) == first
+    assert not _ or not log("copy device")  # (both plans are kept)
+""")
+
+
 def test_a_requested_halo_is_not_widened(run):
     """A halo of 16 that the caller asked for stays 16, in any precision and
     after an autotune; one left free widens, and is free again with 0."""
