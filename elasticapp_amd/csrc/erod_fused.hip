@@ -200,9 +200,9 @@ namespace erod {
   // over the state twice more (calls on one rod of 300, us: 1 step 16 whole and
   // 25 in pieces, 8 steps 44 and 44, 16 steps 75 and 63, 100 steps 402 and 274).
   // Results are the same, bit by bit; FP32-bulk's depend on where a launch ends,
-  // so its rods stay whole.  (Batches with rods of 513 to 1,024 elements would gain more,
-  // 13.6 -> 3.5 for 20 of them, but take 1024 lanes by promise: an autotune, or
-  // a request for pieces, has them faster.)
+  // so its rods stay whole.  (Batches with rods of 513 to 1,024 elements would
+  // gain more, 13.6 -> 3.5 for 20 of them, but erod_set_fused_config documents
+  // 1024 lanes for them: an autotune, or a request for pieces, has them faster.)
   // A shape the autotuner chose is taken again while it stays feasible (a
   // replan after rods changed length keeps it, with its second group).  Tuned
   // for FP32-bulk, 128 lanes may have two elements per thread in one wave, for
@@ -421,7 +421,8 @@ namespace erod {
   // 64, a launch taking as many steps.  Until then wider halos cost no time,
   // and longer launches save it (a launch costs 20 us beside its steps): 24
   // rods of 2,500 to 6,000 elements, us a step FP32-bulk 3.75 -> 2.31, FP64 7.7
-  // -> 4.95; 3 rods of 1,200 to 1,500 2.2 -> 1.64 and 3.6 -> 2.90.  FP32-bulk's runs stay `halo` / 2 steps, so results don't depend on it.
+  // -> 4.95; 3 rods of 1,200 to 1,500 2.2 -> 1.64 and 3.6 -> 2.90.  FP32-bulk's
+  // runs stay `halo` / 2 steps, so results don't depend on it.
   static uint64_t wide_halo(const erod_batch* b, int main_shape, uint64_t pcap, uint64_t halo) {
     const uint64_t step = halo / 2, cap = uint64_t(fused_shape_lanes(main_shape));
     uint64_t wide = halo, whole = 0;
@@ -588,9 +589,10 @@ namespace erod {
     gs.n_segs = segs.size() - uncut;
     gs.n_seg_rods = seg_rods.size();
     // FP32-bulk's merged half steps end every halo / 2 steps, wherever launches
-    // end; a launch holds two such runs (three for a halo of 3, more in a wide one).  13 launches per 100 steps (halo 16)
-    // became 7: 24 rods of 2,500 to 6,000 elements 6.05 -> 5.08 us a step
-    // (FP32-bulk), 2,048 ragged rods 29.6 -> 28.0 (FP64, long rods in pieces)
+    // end; a launch holds two such runs (three for a halo of 3, more in a wide
+    // one).  13 launches per 100 steps (halo 16) became 7: 24 rods of 2,500 to
+    // 6,000 elements 6.05 -> 5.08 us a step (FP32-bulk), 2,048 ragged rods 29.6
+    // -> 28.0 (FP64, long rods in pieces)
     gs.run_steps = int(halo / 2);
     gs.max_steps = int(wide / (halo / 2)) * gs.run_steps;
     if (segs.empty()) gs.shape = -1;

@@ -901,8 +901,6 @@ namespace erod {
       } else if constexpr (kHold) {
         const uint64_t s = slot[0];
         load_const<R>(C, s, E, !(kk[0] == nn[0] - 1) && !pad[0], H);
-#pragma unroll
-        for (int c = 0; c < 3; ++c) H.iJ[c] = C.iJ[c * E + s];
         H.il0 = step64::divisor<true>(H.l0).r;
         H.iD0 = step64::divisor<true>(H.D0).r;
         // the damping products, formed as every step would form them
@@ -945,8 +943,9 @@ namespace erod {
       if constexpr (kRuns && P == 1) asm volatile("" : "+v"(run), "+v"(rest));
       // FP64: the half step that closes a step turns the directors as the one
       // that opens the next does (same w, same dt), by one rotation: 885
-      // VALU instructions a step instead of 970; 500 steps of 1,024 rods of 64
-      // elements 1.50 -> 1.34 ms, 20 of one rod of 100 elements 75 -> 69 us.
+      // VALU instructions a step instead of 970 (873 since); 500 steps of 1,024
+      // rods of 64 elements 1.50 -> 1.34 ms (1.25 since), 20 of one rod of 100
+      // elements 75 -> 69 us (55 since).
       // With more elements per thread the rotations would be spilled.
       constexpr bool kTurn = !kCache && P == 1;
       step64::Rotation turn;

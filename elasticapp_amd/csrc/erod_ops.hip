@@ -511,9 +511,9 @@ namespace erod {
     // ---- several whole steps in one launch -----------------------------------------
 
     // Steps per launch of k_steps: more of them amortise its loads and launch,
-    // and cost 2 slots of a workgroup's 256 each.  Measured with 4 / 8 / 12 / 16:
-    // 18.1 / 17.9 / 17.0 / 16.9 us a step at 248,188 elements, 60.9 / 55.8 /
-    // 54.8 / 55.3 at 992,754.  One workgroup has nothing to recompute.
+    // and cost 2 slots of a workgroup's 256 each.  Measured with 4 / 8 / 12 / 16 /
+    // 20: 12.8 / 12.1 / 11.3 / 11.0 / 10.9 us a step at 248,188 elements, 46.5 /
+    // 39.7 / 37.5 / 38.1 / 38.8 at 992,754.  One workgroup has nothing to recompute.
     constexpr uint64_t kStepsPerLaunch = 12, kStepsOneBlock = 100;
 
     // x, v, Q, w: the state a launch of k_steps reads or writes
@@ -549,10 +549,11 @@ namespace erod {
     // workgroup reads `in` and writes `out`, two copies of the state, so that
     // none writes what another reads.  A block of at most kThreads slots is
     // one workgroup (left = 0, own = its slots), in place, for any nsteps.
-    // Bound by VALU issue like the fused FP64 kernel (190 VGPRs, two workgroups
-    // per CU); constants stay in registers for the launch.  17.0 us a step at
-    // 248,188 elements against 209 with a pass per operator, 5.3 against 113 on
-    // one rod of 100 elements (46 launches a step before).
+    // Bound by VALU issue like the fused FP64 kernel (208 VGPRs, two workgroups
+    // per CU, 876 VALU instructions per wave and step); constants stay in
+    // registers for the launch.  11.3 us a step at 248,188 elements against 209
+    // with a pass per operator, 3.1 against 113 on one rod of 100 elements (46
+    // launches a step before).
     __global__ void __launch_bounds__(kThreads) k_steps(State in, State out, Lines f, const uint8_t* __restrict__ is_ghost,
                                                         const uint32_t* __restrict__ rod_of,
                                                         const RodInfo* __restrict__ rods, Env env, bool damped, double dt,

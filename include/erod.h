@@ -181,8 +181,9 @@ int erod_set_rod_time(erod_batch* b, const double* time_per_rod);
  * otherwise; FP32-bulk batches that fill the device take two elements per
  * thread in 128 lanes for rods of up to 128 elements, in 512 for rods of up to
  * 256; small FP64 batches whose longest rod has 257 to 512 elements take 256
- * lanes, but for calls of launches shorter than 16 steps); rods longer than
- * the tile run as pieces (erod_set_fused_pieces).  Results do not depend on the
+ * lanes, but for calls of launches shorter than 16 steps, a requested halo
+ * below 6 or above 96, and servers' pools); rods longer than the tile run as
+ * pieces (erod_set_fused_pieces).  Results do not depend on the
  * shape, bit for bit; FP32-bulk's not on one that leaves the same rods whole. */
 int erod_set_fused_config(erod_batch* b, int lanes_per_tile, int elements_per_thread, int steps_per_launch);
 int erod_get_fused_config(const erod_batch* b, int* lanes_per_tile, int* elements_per_thread, int* steps_per_launch);
