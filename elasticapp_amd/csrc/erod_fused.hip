@@ -759,10 +759,11 @@ namespace erod {
     // default_shape).  FP32-bulk rounds a rod that is cut by its halo: where 512
     // lanes hold every rod, shapes that cut some are not tried, so that a tuned
     // batch returns what an untuned one does, and not what the trials' times
-    // happen to decide.  (Pieces with wide halos would be faster: passes of 11
-    // rods of 105 to 258 elements 1.09 ms against 1.22, of 15 rods of 25 to 314
-    // 0.65 against 0.73.  With longer rods, beside which whole ones run in
-    // 1024 lanes, 2.9 against 4.3 for 70 of 44 to 718, they are tried.)
+    // happen to decide.  (Pieces with wide halos would be faster for few rods,
+    // ms a pass: 21 of 76 to 355 elements 1.40 against 2.02, 15 of 80 to 349 1.01
+    // and 1.43, 11 of 105 to 258 1.11 and 1.23; slower for many, 476 of 17 to 287
+    // 3.68 and 3.42.  With longer rods, beside which whole ones run in 1024
+    // lanes, 2.9 against 4.3 for 70 of 44 to 718, they are tried.)
     const uint64_t longest = extent(b).longest;
     const bool keep_whole = precision != EROD_FP64 && b->plan.seg_lanes == 0 && longest <= 512;
     auto has_registers = [&](int si) { return si != kShape128x2 || precision != EROD_FP64; };
