@@ -220,6 +220,9 @@ int erod_get_fused_pieces(const erod_batch* b, int* lanes_per_tile, int* element
                           uint64_t* tiles, uint64_t* pieces);
 /* Times every feasible tile shape on `trial_steps` steps from a snapshot of
  * the state (restored afterwards) and keeps the fastest; reports its ms/step.
+ * FP32-bulk, which rounds a rod that is cut otherwise than a whole one, tries
+ * only shapes that leave the rods whole where 512 lanes hold each of them and
+ * no pieces' shape was requested.
  * No counterpart in the reference (its blocks are sized by a fixed policy,
  * elastica/Simulator/Configuration/ModuleConfiguration/BlockingPolicy.hpp:291-321). */
 int erod_autotune_fused(erod_batch* b, int precision, int trial_steps, double* best_ms_per_step);
